@@ -75,6 +75,10 @@ SIGNATURES = {
     "dmad_attn_jvp_fwd": (_INT, [_INT, _INT, _I64, _I64, _I64, _I64, _I64, _I64,
                                  _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
                                  _P, _P, _I64P, _P, _P, _F, _P, _SZ, _P]),
+    "dmad_attn_fwd_split_bytes": (_INT, [_INT, _INT, _I64, _I64, _I64, _I64, _I64, _I64, _SZP]),
+    "dmad_attn_jvp_fwd_split": (_INT, [_INT, _INT, _I64, _I64, _I64, _I64, _I64, _I64,
+                                       _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
+                                       _P, _P, _I64P, _P, _P, _F, _P, _SZ, _P, _SZ, _P]),
     "dmad_attn_jvp_fwd_magi": (_INT, [_INT, _INT, _I64, _I64, _I64, _I64, _I64, _I64,
                                       _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
                                       _P, _P, _I64P, _P, _P, _F,
@@ -180,6 +184,15 @@ def stream_ptr(device: torch.device) -> int:
 def fwd_workspace_bytes(mode: int, B: int, H: int, Lk: int, Dqk: int, Dv: int) -> int:
     n = ctypes.c_size_t(0)
     check(lib().dmad_attn_fwd_workspace_bytes(mode, B, H, Lk, Dqk, Dv, ctypes.byref(n)))
+    return int(n.value)
+
+
+@functools.lru_cache(maxsize=1024)
+def fwd_split_bytes(dtype: int, mode: int, B: int, H: int, Lq: int, Lk: int, Dqk: int, Dv: int) -> int:
+    """Bytes of fp32 partials with which a dense forward splits its last query tiles over
+    their keys (0: it runs every tile whole)."""
+    n = ctypes.c_size_t(0)
+    check(lib().dmad_attn_fwd_split_bytes(dtype, mode, B, H, Lq, Lk, Dqk, Dv, ctypes.byref(n)))
     return int(n.value)
 
 

@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "split.h"
 
 namespace dmad {
 
@@ -72,6 +73,7 @@ struct FwdParams {
   const int* task_qtile;  // [T]
   int G, R, T;
   int xcd_order;  // dense kernels: work items contiguous per XCD (common.h)
+  SplitParams sp;  // split launches of attn_fwd32_kernel (split.h)
 };
 
 // One (query group, 128-query tile) task of the block-sparse forward: group

@@ -30,6 +30,7 @@
 // Every MFMA's LDS operand is read four operands ahead.
 #pragma once
 #include "attn_fwd.h"
+#include "split.h"
 
 namespace dmad {
 
@@ -132,7 +133,11 @@ __device__ __forceinline__ void stage_store(const lds_char_t* region, int k, int
 // Waves per SIMD: one at D = 128 and 256 (the JVP modes hold 416-468
 // registers); two at D = 64, four for its dense plain forward (128 registers,
 // 32 KiB of LDS per workgroup; 1-2% faster than two, bitwise equal).
-template <typename T, int MODE, bool MAGI = false, int DH = 128>
+//
+// SPLIT (64- and 128-wide heads, dense): the last work items of the grid run in
+// pieces of their key range (split.h); a piece sees its keys as the whole
+// sequence and writes O~ / l, C~ / l, its logsumexp and mu as fp32 partials.
+template <typename T, int MODE, bool MAGI = false, int DH = 128, bool SPLIT = false>
 __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2) : 1) void attn_fwd32_kernel(
     FwdParams p) {
   using C = Fwd32Cfg<MODE, DH>;
@@ -158,7 +163,20 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   int bh, qt, ntiles, chunk = 0;
   int q_lo = 0, q_hi = p.Lq;  // rows this workgroup stores
   int r_beg = 0, r_end = 0;   // key ranges of the group (MAGI)
-  if constexpr (MAGI) {
+  int lk = p.Lk, key0 = 0;    // keys of this workgroup (SPLIT: of its piece), the first one's row
+  int part_slot = -1;         // SPLIT: partial block of this piece
+  static_assert(!SPLIT || (!MAGI && C::CHUNKS == 1 && DVC == D), "split launches: dense, all of V in one workgroup");
+  if constexpr (SPLIT) {
+    const int nqt = (p.Lq + C::BM - 1) / C::BM;
+    const SplitWork w = split_work(p.sp, p.xcd_order, (p.Lk + BN - 1) / BN);
+    if (w.item < 0) return;
+    bh = w.item / nqt;
+    qt = w.item - bh * nqt;
+    ntiles = w.end - w.beg;
+    key0 = w.beg * BN;
+    lk = min(p.Lk - key0, ntiles * BN);
+    if (w.piece >= 0) part_slot = w.slot;
+  } else if constexpr (MAGI) {
     int work = xcd_remap(blockIdx.x, p.T * p.B * p.H * C::CHUNKS);
     if constexpr (C::CHUNKS > 1) {
       chunk = work % C::CHUNKS;  // the chunks of one task are adjacent work items
@@ -219,10 +237,14 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   }
 
   // ---- key-side resources and per-lane request offsets (tile independent)
-  const uint32_t k_bytes = (uint32_t)(((int64_t)(p.Lk - 1) * p.k_sl + D) * 2);
+  const uint32_t k_bytes = (uint32_t)(((int64_t)(lk - 1) * p.k_sl + D) * 2);
   // V (Vd) resources start at this workgroup's column chunk
-  const uint32_t v_bytes = (uint32_t)(((int64_t)(p.Lk - 1) * p.v_sl + DVC) * 2);
-  const int64_t khead = b * p.k_sb + h * p.k_sh, vhead = b * p.v_sb + h * p.v_sh + chunk * DVC;
+  const uint32_t v_bytes = (uint32_t)(((int64_t)(lk - 1) * p.v_sl + DVC) * 2);
+  int64_t khead = b * p.k_sb + h * p.k_sh, vhead = b * p.v_sb + h * p.v_sh + chunk * DVC;
+  if constexpr (SPLIT) {
+    khead += (int64_t)key0 * p.k_sl;
+    vhead += (int64_t)key0 * p.v_sl;
+  }
   const __amdgpu_buffer_rsrc_t rk = make_rsrc((const char*)p.k + khead * 2, k_bytes);
   const __amdgpu_buffer_rsrc_t rv = make_rsrc((const char*)p.v + vhead * 2, v_bytes);
   __amdgpu_buffer_rsrc_t rtk = rk, rtv = rv;
@@ -412,7 +434,9 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   // 16 (v >> 3) + 8 half + (v & 7); P~, H~ are packed as the B operands of the
   // two 16-key chunks.
   constexpr int NMICRO = 18;
-  float m_i = -__builtin_inff(), l_i = 0.f, r_i = 0.f;
+  // a piece starts from a finite maximum, so that a row all of whose keys in it
+  // score -inf has l = 0 there rather than NaN
+  float m_i = SPLIT ? -3.0e38f : -__builtin_inff(), l_i = 0.f, r_i = 0.f;
   struct Soft {
     float mx, alpha, neg_m, ls, rs, pv;
     float hv;
@@ -548,7 +572,7 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
     } else {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        if (i * BN + 16 * (v >> 3) + 8 * half + (v & 7) >= p.Lk) sc[v] = -__builtin_inff();
+        if (i * BN + 16 * (v >> 3) + 8 * half + (v & 7) >= lk) sc[v] = -__builtin_inff();
       }
     }
     Soft sm;
@@ -644,6 +668,35 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   const float inv_lh = kHScaled ? inv_l : inv_l * p.scale;  // 1 / l, with the scale H~ left out
   float mu = 0.f;
   if constexpr (C::JVP) mu = (r_i + other_half(r_i)) * inv_lh;
+  if constexpr (SPLIT) {
+    if (part_slot >= 0) {
+      using P = FwdPart<D, C::JVP>;
+      float* const part = p.sp.part + (int64_t)part_slot * P::FLOATS;
+      float* const tile = part + wave * P::NT * P::TILE;
+      const float keep_l = l == 0.f ? 0.f : inv_l, keep_lh = l == 0.f ? 0.f : inv_lh;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          f32x4_t ov, cv;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            ov[e] = oacc[d][4 * jj + e] * keep_l;
+            if constexpr (C::JVP) cv[e] = cacc[d][4 * jj + e] * keep_lh;
+          }
+          split_put<D>(tile, lane, d, jj, ov);
+          if constexpr (C::JVP) split_put<D>(tile + P::TILE, lane, d, jj, cv);
+        }
+        if constexpr (kAccAgpr) __builtin_amdgcn_sched_barrier(0);
+      }
+      if (half == 0) {
+        float* const st = part + P::STATS + wave * 64 + col;
+        st[0] = exp_base<T>(m_i) + __builtin_log2f(l);
+        if constexpr (C::JVP) st[32] = l == 0.f ? 0.f : mu;
+      }
+      return;
+    }
+  }
   // O (Od) resources start at this workgroup's column chunk
   const int64_t obase = b * p.o_sb + h * p.o_sh + chunk * DVC;
   const uint32_t o_bytes = (uint32_t)(((int64_t)(p.Lq - 1) * p.o_sl + DVC) * 2);

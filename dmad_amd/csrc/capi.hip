@@ -263,6 +263,45 @@ FwdPlan plan_fwd(int dtype, int mode, int64_t magi_tasks, int64_t B, int64_t H, 
   return pl;
 }
 
+// Costs of attn_fwd32_kernel's workgroups for plan_split. Measured (bf16, H=12,
+// graph replays, the second number split): plain, 1560 x 7801 tokens, 156 tiles on
+// 512 slots 115 -> 92 us in three pieces; plain, 10920 tokens, 8 tiles after two
+// full rounds 748 -> 657 us; JVP, 6240 tokens, 76 tiles after two rounds 660 ->
+// 578 us; JVP, 999 tokens of two heads 37 -> 24.5 us in four pieces (eight: 27.4).
+// A launch whose tiles fill more than half of the chip does not split in the JVP
+// modes: 156 tiles of 1560 keys, 57-65 us whole, took 67 us in pieces of 33 and 16
+// steps (41 MB of partials).
+dmad::SplitCost fwd_split_cost(int mode, int64_t D) {
+  const bool jvp = mode != DMAD_FWD_PLAIN;
+  if (D == 128) {
+    if (jvp) return {1, 1.0f, 0.f, 12.f, dmad::FwdPart<128, true>::FLOATS * 4};
+    return {2, 0.42f, 0.6f, 7.f, dmad::FwdPart<128, false>::FLOATS * 4};
+  }
+  if (jvp) return {2, 0.55f, 0.8f, 8.f, dmad::FwdPart<64, true>::FLOATS * 4};
+  return {4, 0.3f, 0.6f, 6.f, dmad::FwdPart<64, false>::FLOATS * 4};
+}
+
+// The split of a dense forward's last query tiles over their keys. Both JVP
+// modes split alike (with the full JVP's costs), so that O does not depend on
+// whether Kd = Vd = 0 was stated; they split no key range of 512 or fewer, which
+// the two-workgroups-per-CU kernel serves, and up to 2048 keys, where that kernel
+// would run two tiles per CU, only launches that leave CUs without a tile.
+dmad::SplitPlan plan_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk,
+                               int64_t Dv) {
+  const int64_t items = (Lq + 127) / 128 * B * H, steps = (Lk + 31) / 32;
+  dmad::SplitPlan none;
+  none.whole = none.grid = items;
+  if (dtype == DMAD_F32 || !dmad::fwd32_supported((int)Dqk, (int)Dv)) return none;
+  if (mode != DMAD_FWD_PLAIN && (steps <= 16 || (steps <= kX2MaxKeyTiles && items >= dmad::kSplitCus))) return none;
+  return dmad::plan_split(items, steps, fwd_split_cost(mode, Dqk));
+}
+
+dmad::FwdLaunchFn pick_fwd_split(int dtype, int64_t d, int mode) {
+  if (dtype == DMAD_BF16) return dmad::fwd32_split_select<__bf16>(mode, (int)d);
+  if (dtype == DMAD_F16) return dmad::fwd32_split_select<_Float16>(mode, (int)d);
+  return nullptr;
+}
+
 // Block-sparse tables of dmad_attn_jvp_fwd_magi (device pointers).
 struct MagiArgs {
   const int32_t *q_ranges, *k_ranges, *qk_map, *task_group, *task_qtile;
@@ -470,8 +509,8 @@ BwdPlan plan_bwd_ws(int dtype, bool full, bool tgrad, int64_t B, int64_t H, int6
 int fwd_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv, const void* q,
              const void* k, const void* v, const void* tq, const void* tk, const void* tv, const int64_t q_strides[4],
              const int64_t k_strides[4], const int64_t v_strides[4], void* o, void* to, const int64_t o_strides[4],
-             float* lse, float* mu, float sm_scale, void* workspace, size_t workspace_bytes, void* stream,
-             const MagiArgs* mg) {
+             float* lse, float* mu, float sm_scale, void* workspace, size_t workspace_bytes, void* split_ws,
+             size_t split_bytes, void* stream, const MagiArgs* mg) {
   if (dtype != DMAD_BF16 && dtype != DMAD_F16 && dtype != DMAD_F32)
     return fail(DMAD_ERR_UNSUPPORTED, "unsupported dtype code %d", dtype);
   if (mode < DMAD_FWD_PLAIN || mode > DMAD_FWD_JVP_KV_TANGENT_ZERO) return fail(DMAD_ERR_INVALID, "unknown mode %d", mode);
@@ -510,6 +549,7 @@ int fwd_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, 
   if (need > 0 && (workspace == nullptr || (int64_t)workspace_bytes < need))
     return fail(DMAD_ERR_WORKSPACE, "workspace needs %lld bytes, got %lld", (long long)need, (long long)workspace_bytes);
   if (((uintptr_t)workspace & 255) != 0) return fail(DMAD_ERR_INVALID, "workspace must be 256-byte aligned");
+  if (((uintptr_t)split_ws & 255) != 0) return fail(DMAD_ERR_INVALID, "the split workspace must be 256-byte aligned");
   const int64_t dvp = Dv < 32 ? 32 : Dv, lkp = round_up(Lk, kLkAlign);
   if (dvp * lkp * 2 >= kMaxHeadBytes) return fail(DMAD_ERR_UNSUPPORTED, "Lk too large");
 
@@ -518,6 +558,14 @@ int fwd_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, 
                          : mg                                ? pick_fwd_magi(dtype, Dqk, Dv, mode)
                                                              : pick_fwd(dtype, Dqk, Dv, mode);
   if (fn == nullptr) return fail(DMAD_ERR_UNSUPPORTED, "no kernel for Dqk=%lld Dv=%lld", (long long)Dqk, (long long)Dv);
+
+  // with room for the partials, the last query tiles run in pieces of their keys
+  dmad::SplitPlan sp;
+  if (split_ws != nullptr && mg == nullptr) {
+    sp = plan_fwd_split(dtype, mode, B, H, Lq, Lk, Dqk, Dv);
+    if (sp.rest == 0 || (int64_t)split_bytes < sp.bytes) sp = dmad::SplitPlan{};
+    else if ((fn = pick_fwd_split(dtype, Dqk, mode)) == nullptr) return fail(DMAD_ERR_UNSUPPORTED, "no split kernel");
+  }
 
   hipStream_t s = (hipStream_t)stream;
   const int BH = (int)(B * H);
@@ -580,8 +628,9 @@ int fwd_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, 
     p.R = (int)mg->R;
     p.T = (int)mg->T;
   }
-  if (plan.grid >= ((int64_t)1 << 31)) return fail(DMAD_ERR_UNSUPPORTED, "grid too large");
-  const int64_t grid = plan.grid;
+  const int64_t grid = sp.rest > 0 ? sp.grid : plan.grid;
+  if (grid >= ((int64_t)1 << 31)) return fail(DMAD_ERR_UNSUPPORTED, "grid too large");
+  if (sp.rest > 0) p.sp = dmad::SplitParams{(int)sp.whole, (int)sp.rest, sp.n, sp.len, (float*)split_ws};
   p.xcd_order = plan.xcd_order;  // block order (common.h)
   mark(0, false, s);
   e = fn(p, (int)grid, s);
@@ -986,7 +1035,26 @@ int dmad_attn_jvp_fwd(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int
                       void* to, const int64_t o_strides[4], float* lse, float* mu, float sm_scale, void* workspace,
                       size_t workspace_bytes, void* stream) {
   return fwd_impl(dtype, mode, B, H, Lq, Lk, Dqk, Dv, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to,
-                  o_strides, lse, mu, sm_scale, workspace, workspace_bytes, stream, nullptr);
+                  o_strides, lse, mu, sm_scale, workspace, workspace_bytes, nullptr, 0, stream, nullptr);
+}
+
+int dmad_attn_fwd_split_bytes(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk,
+                              int64_t Dv, size_t* bytes) {
+  if (bytes == nullptr) return fail(DMAD_ERR_INVALID, "bytes: null pointer");
+  if (mode < DMAD_FWD_PLAIN || mode > DMAD_FWD_JVP_KV_TANGENT_ZERO) return fail(DMAD_ERR_INVALID, "unknown mode %d", mode);
+  if (B < 0 || H < 0 || Lq < 0 || Lk < 0 || !head_dim_ok(Dqk) || !head_dim_ok(Dv)) return fail(DMAD_ERR_INVALID, "bad sizes");
+  *bytes = (size_t)plan_fwd_split(dtype, mode, B, H, Lq, Lk, Dqk, Dv).bytes;
+  return ok();
+}
+
+int dmad_attn_jvp_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv,
+                            const void* q, const void* k, const void* v, const void* tq, const void* tk,
+                            const void* tv, const int64_t q_strides[4], const int64_t k_strides[4],
+                            const int64_t v_strides[4], void* o, void* to, const int64_t o_strides[4], float* lse,
+                            float* mu, float sm_scale, void* workspace, size_t workspace_bytes, void* split_ws,
+                            size_t split_bytes, void* stream) {
+  return fwd_impl(dtype, mode, B, H, Lq, Lk, Dqk, Dv, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to,
+                  o_strides, lse, mu, sm_scale, workspace, workspace_bytes, split_ws, split_bytes, stream, nullptr);
 }
 
 int dmad_attn_jvp_fwd_magi(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv,
@@ -1006,7 +1074,7 @@ int dmad_attn_jvp_fwd_magi(int dtype, int mode, int64_t B, int64_t H, int64_t Lq
     return fail(DMAD_ERR_INVALID, "block-sparse tables: null pointer");
   const MagiArgs mg{q_ranges, k_ranges, qk_map, task_group, task_qtile, G, R, T};
   return fwd_impl(dtype, mode, B, H, Lq, Lk, Dqk, Dv, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to,
-                  o_strides, lse, mu, sm_scale, workspace, workspace_bytes, stream, &mg);
+                  o_strides, lse, mu, sm_scale, workspace, workspace_bytes, nullptr, 0, stream, &mg);
 }
 
 int dmad_attn_fwd(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv, const void* q,

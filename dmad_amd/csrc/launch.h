@@ -26,6 +26,13 @@ FwdLaunchFn fwd32_select(int mode, int d);
 template <> FwdLaunchFn fwd32_select<__bf16>(int, int);
 template <> FwdLaunchFn fwd32_select<_Float16>(int, int);
 
+// attn_fwd32_kernel with the last work items split over their keys, and the
+// kernel that combines their pieces (64- and 128-wide heads; FwdParams::sp).
+template <typename T>
+FwdLaunchFn fwd32_split_select(int mode, int d);
+template <> FwdLaunchFn fwd32_split_select<__bf16>(int, int);
+template <> FwdLaunchFn fwd32_split_select<_Float16>(int, int);
+
 // Two-workgroups-per-CU forward (attn_fwd32_x2_kernel; mode kFwdJvpQOnly,
 // 128-wide heads): one workgroup per 128-query tile.
 template <typename T>

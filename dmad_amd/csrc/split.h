@@ -1,0 +1,266 @@
+// Splitting the last work items of a launch over the loop they run.
+//
+// The attention passes give one workgroup one work item: a tile of queries (or
+// keys) of one head, walked against all keys (or queries). A grid that is not a
+// whole number of rounds over the chip leaves most CUs idle in its last round:
+// 588 items of one workgroup per CU run 2.3 rounds of work in the time of 3, and
+// 156 items keep 100 of the 256 CUs idle throughout. A split launch runs the
+// items of the full rounds as before and cuts each of the `rest` items after them
+// into `n` pieces along its loop. A piece writes its fp32 accumulators to a
+// partial buffer, and a second, small kernel sums an item's pieces in a fixed
+// order (no atomics: repeated calls agree bit for bit) and writes the outputs.
+// What a launch does is decided once per shape on the host (plan_split) from the
+// items, the steps of an item's loop and the costs of the kernel that runs it.
+#pragma once
+#include "common.h"
+
+namespace dmad {
+
+// Kernel arguments of a split launch (rest == 0: an ordinary launch).
+struct SplitParams {
+  int whole;    // work items [0, whole) run whole, one workgroup each
+  int rest;     // work items [whole, whole + rest) run in pieces
+  int n;        // pieces per split item
+  int len;      // steps of pieces 0 .. n - 2; the last piece takes what is left
+  float* part;  // partials, [rest][n] blocks
+};
+
+// What this workgroup of a split launch runs.
+struct SplitWork {
+  int item;      // work item; -1: none (a padding workgroup of the last ids)
+  int piece;     // -1: the whole item
+  int slot;      // (item - whole) n + piece: index of the piece's partial block
+  int beg, end;  // steps of the item's loop
+};
+
+// Workgroups of a split launch: the whole items, then per XCD its share of the
+// split items, piece-major, so that the equal, longer pieces start first and a
+// shorter last piece fills the gaps they leave, and an item's pieces (which read
+// the same rows of one head) share an L2.
+__host__ __device__ inline int64_t split_grid(int64_t whole, int64_t rest, int64_t n) {
+  return whole + 8 * ((rest + 7) / 8) * n;
+}
+
+__device__ __forceinline__ SplitWork split_work(const SplitParams& sp, int xcd_order, int steps) {
+  const int bid = (int)blockIdx.x;
+  if (bid < sp.whole) return SplitWork{xcd_order ? xcd_remap(bid, sp.whole) : bid, -1, 0, 0, steps};
+  const int id = bid - sp.whole, xcd = id & 7, k = id >> 3;
+  const int per = sp.rest >> 3, rem = sp.rest & 7;
+  const int first = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
+  const int mine = per + (xcd < rem ? 1 : 0);  // split items of this XCD
+  if (mine == 0 || k >= mine * sp.n) return SplitWork{-1, 0, 0, 0, 0};
+  const int piece = k / mine, j = first + (k - piece * mine);
+  const int beg = piece * sp.len;
+  return SplitWork{sp.whole + j, piece, j * sp.n + piece, beg, piece + 1 < sp.n ? beg + sp.len : steps};
+}
+
+// Partial block of one piece: per wave and tensor, the wave's 32 x D accumulator
+// tile in the 32x32 MFMA layout (lane: row lane % 32, columns 32 d + 8 jj +
+// 4 (lane / 32) + 0..3), 16 bytes per lane and (d, jj), so every store and load
+// instruction moves 1 KiB in a row.
+template <int D>
+__host__ __device__ constexpr int split_tile_floats() { return 32 * D; }
+template <int D>
+__device__ __forceinline__ void split_put(float* tile, int lane, int d, int jj, f32x4_t v) {
+  *(f32x4_t*)(tile + ((4 * d + jj) * 64 + lane) * 4) = v;
+}
+template <int D>
+__device__ __forceinline__ f32x4_t split_get(const float* tile, int lane, int g) {
+  return *(const f32x4_t*)(tile + (g * 64 + lane) * 4);
+}
+
+// ---------------------------------------------------------------- host: the plan
+// Costs of one kernel of a split launch, in microseconds on an MI355X.
+struct SplitCost {
+  int occ;          // workgroups that fit a CU
+  float step;       // one step of the loop, one workgroup per CU
+  float shared;     // factor on a step's time per further workgroup on the CU
+  float fixed;      // a workgroup's time outside its loop
+  int part_bytes;   // partial block of one piece
+};
+struct SplitPlan {
+  int64_t whole = 0, rest = 0, grid = 0, bytes = 0;
+  int n = 1, len = 0;
+};
+
+constexpr int kSplitCus = 256;
+constexpr int kSplitMaxPieces = 64;
+
+// Time of `a` workgroups of la steps followed by `b` of lb <= la, dealt to the
+// free slots in that order.
+inline double split_makespan(const SplitCost& k, int64_t a, double la, int64_t b, double lb) {
+  const int64_t total = a + b;
+  if (total == 0) return 0.;
+  const int64_t per = (total + kSplitCus - 1) / kSplitCus;
+  const int occ = (int)(per < k.occ ? per : k.occ);  // workgroups sharing a CU
+  const double step = k.step * (1. + k.shared * (occ - 1));
+  const double ta = la * step + k.fixed, tb = lb * step + k.fixed;
+  const int64_t slots = (int64_t)kSplitCus * occ;
+  double t = (double)(a / slots) * ta;  // full rounds of the long ones
+  const int64_t busy = a % slots;       // slots busy for another ta
+  if (b == 0) return t + (busy ? ta : 0.);
+  double best = 0.;
+  for (int64_t r = 1;; ++r) {  // r short ones in a row on a free slot
+    const double end = (double)r * tb;
+    const int64_t after = end > ta ? (int64_t)((end - ta) / tb) : 0;
+    if ((slots - busy) * r + busy * after >= b) {
+      best = end;
+      break;
+    }
+  }
+  if (busy && best < ta) best = ta;
+  return t + best;
+}
+
+// How to run `items` work items of `steps` steps: in full rounds, then the rest in
+// the pieces that finish soonest by the costs above, where that saves at least a
+// twentieth of the launch. The partials are written and read once, at about
+// 3.3 TB/s, by a second kernel that takes 5 us at least (all measured).
+inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k) {
+  SplitPlan pl;
+  pl.whole = items;
+  pl.grid = items;
+  const int64_t slots = (int64_t)kSplitCus * k.occ, rest = items % slots, rounds = items / slots;
+  if (rest == 0 || steps < 4) return pl;
+  const double round = (1. + k.shared * (k.occ - 1)) * k.step * (double)steps + k.fixed;
+  const double as_is = split_makespan(k, rest, (double)steps, 0, 0.);
+  double best = as_is - 0.05 * (as_is + (double)rounds * round);
+  for (int64_t n = 2; n <= kSplitMaxPieces && 2 * n <= steps; ++n) {
+    const double extra = 5. + 2. * (double)(rest * n) * k.part_bytes / 3.3e6;
+    const int64_t even = (steps + n - 1) / n;
+    // the shorter last piece runs in the slots the n - 1 long ones leave free
+    const int64_t left = slots - (n - 1) * rest;
+    int64_t lens[2] = {even, 0};
+    if (left > 0 && left < rest) {
+      const int64_t q = (rest + left - 1) / left;
+      lens[1] = (steps * q + (n - 1) * q) / ((n - 1) * q + 1);
+    }
+    for (const int64_t a : lens) {
+      const int64_t b = steps - (n - 1) * a;
+      if (a < 1 || b < 1 || b > a) continue;
+      const double t = split_makespan(k, (n - 1) * rest, (double)a, rest, (double)b) + extra;
+      if (t < best) {
+        best = t;
+        pl.n = (int)n;
+        pl.len = (int)a;
+      }
+    }
+  }
+  if (pl.n > 1) {
+    pl.whole = items - rest;
+    pl.rest = rest;
+    pl.grid = split_grid(pl.whole, rest, pl.n);
+    pl.bytes = rest * pl.n * k.part_bytes;
+  }
+  return pl;
+}
+
+// ---------------------------------------------------------------- forward
+// Partial block of the forward: [4 waves][O (, C)][32 x D], then per wave
+// [lse2, mu][32 rows]. O = O~ / l and C = C~ / l of the piece's keys, lse2 its
+// log2-domain logsumexp.
+template <int D, bool JVP>
+struct FwdPart {
+  static constexpr int NT = JVP ? 2 : 1;
+  static constexpr int TILE = split_tile_floats<D>();
+  static constexpr int STATS = 4 * NT * TILE;
+  static constexpr int FLOATS = STATS + 4 * 2 * 32;
+};
+
+struct FwdCombineParams {
+  SplitParams sp;
+  void* o;
+  void* to;
+  float* lse;
+  float* mu;
+  int64_t o_sb, o_sh, o_sl;
+  int H, Lq;
+};
+
+// One workgroup per wave tile (32 queries) of a split item; thread = (lane of the
+// tile, one of 4 groups of columns). Bound by reading the partials once.
+template <typename T, int D, bool JVP>
+__global__ __launch_bounds__(256) void fwd_combine_kernel(FwdCombineParams p) {
+  using P = FwdPart<D, JVP>;
+  const int item = (int)blockIdx.x >> 2, wave = (int)blockIdx.x & 3;
+  const int lane = lane_id(), col = lane & 31, half = lane >> 5, grp = threadIdx.x >> 6;
+  const int nqt = (p.Lq + 127) / 128;
+  const int work = p.sp.whole + item, bh = work / nqt, qt = work - bh * nqt;
+  const int query = qt * 128 + wave * 32 + col;
+  const float* part = p.sp.part + (int64_t)item * p.sp.n * P::FLOATS;
+  const float* st = part + P::STATS + wave * 64 + col;
+  // pieces are taken U at a time with all of their loads in flight together (the
+  // partials come from other XCDs' workgroups, about a microsecond away); past
+  // the last piece the last one is read again and left out
+  constexpr int U = 4, NG = D / 32;  // NG: 16-byte column groups per thread
+  const int n = p.sp.n;
+  float m = -__builtin_inff();
+  for (int i = 0; i < n; i += 2 * U) {
+    float v[2 * U];
+#pragma unroll
+    for (int u = 0; u < 2 * U; ++u) v[u] = st[(int64_t)min(i + u, n - 1) * P::FLOATS];
+#pragma unroll
+    for (int u = 0; u < 2 * U; ++u) m = fmaxf(m, v[u]);
+  }
+  float w = 0.f, mu = 0.f;
+  f32x4_t o[NG], c[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) o[g] = c[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < n; i += U) {
+    f32x4_t ov[U][NG], cv[U][NG];
+    float lse2[U], mus[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float* pi = part + (int64_t)min(i + u, n - 1) * P::FLOATS;
+      lse2[u] = pi[P::STATS + wave * 64 + col];
+      if constexpr (JVP) mus[u] = pi[P::STATS + wave * 64 + 32 + col];
+      const float* tile = pi + wave * P::NT * P::TILE;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        ov[u][g] = split_get<D>(tile, lane, 4 * g + grp);
+        if constexpr (JVP) cv[u][g] = split_get<D>(tile + P::TILE, lane, 4 * g + grp);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i + u >= n) break;
+      const float wi = fast_exp2(lse2[u] - m);
+      w += wi;
+      if constexpr (JVP) mu += wi * mus[u];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          o[g][e] = fmaf(wi, ov[u][g][e], o[g][e]);
+          if constexpr (JVP) c[g][e] = fmaf(wi, cv[u][g][e], c[g][e]);
+        }
+      }
+    }
+  }
+  if (query >= p.Lq) return;
+  const float inv = 1.0f / w;
+  mu *= inv;
+  const int b = bh / p.H, h = bh - b * p.H;
+  const int64_t off = b * p.o_sb + h * p.o_sh + (int64_t)query * p.o_sl;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const int dc = 32 * g + 8 * grp + 4 * half;
+    float ov[4], tv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      ov[e] = o[g][e] * inv;
+      tv[e] = c[g][e] * inv - mu * ov[e];
+    }
+    *(u32x2_t*)((char*)p.o + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(ov[0], ov[1]), Elem<T>::pack2(ov[2], ov[3])};
+    if constexpr (JVP)
+      *(u32x2_t*)((char*)p.to + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(tv[0], tv[1]), Elem<T>::pack2(tv[2], tv[3])};
+  }
+  if (half == 0 && grp == 0) {
+    const int64_t si = (int64_t)bh * p.Lq + query;
+    p.lse[si] = (m + __builtin_log2f(w)) * 0.6931471805599453f;
+    if constexpr (JVP) p.mu[si] = mu;
+  }
+}
+
+}  // namespace dmad

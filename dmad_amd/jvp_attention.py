@@ -169,6 +169,17 @@ def _backward_workspace(code: int, ws_mode: int, B: int, H: int, Lq: int, Lk: in
     return nat.workspace(base, device)
 
 
+def _split_workspace(nbytes: int, device):
+    """(pointer, size, owner) of the partials of a split launch. The split only saves time:
+    without room for its partials (at most 64 MiB or so) every tile runs whole."""
+    if nbytes == 0:
+        return None, 0, None
+    try:
+        return nat.workspace(nbytes, device)
+    except torch.cuda.OutOfMemoryError:
+        return None, 0, None
+
+
 def _score_slices(bh: int, n_max: int, Lq: int, Lk: int) -> int:
     """(b, h) slices per launch pair, at most n_max: the count whose pairs fill the 256 CUs
     best. A pair of n slices runs n * key tiles key-pass workgroups and n * query-block
@@ -353,13 +364,14 @@ def jvp_attention_forward(q, k, v, tq, tk, tv, sm_scale, need_mu=True):
     mu = torch.empty_like(lse) if tq is not None else None
     lib = nat.lib()
     ws_ptr, ws_size, ws = nat.workspace(_fwd_dense_ws_bytes(q.dtype, mode, B, H, Lk, Dqk, Dv), dev)
+    sp_ptr, sp_size, sp = _split_workspace(nat.fwd_split_bytes(code, mode, B, H, Lq, Lk, Dqk, Dv), dev)
     nat.check(
-        lib.dmad_attn_jvp_fwd(
+        lib.dmad_attn_jvp_fwd_split(
             code, mode, B, H, Lq, Lk, Dqk, Dv,
             nat.ptr(q), nat.ptr(k), nat.ptr(v), nat.ptr(tq), nat.ptr(tk), nat.ptr(tv),
             nat.strides4(q), nat.strides4(k), nat.strides4(v),
             nat.ptr(o), nat.ptr(to), nat.strides4(o), nat.ptr(lse), nat.ptr(mu),
-            float(sm_scale), ws_ptr, ws_size, nat.stream_ptr(dev),
+            float(sm_scale), ws_ptr, ws_size, sp_ptr, sp_size, nat.stream_ptr(dev),
         )
     )
     return o, to, lse, mu

@@ -80,6 +80,28 @@ int dmad_attn_jvp_fwd(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int
                       size_t workspace_bytes, void* stream);
 
 /*
+ * Bytes of partials with which dmad_attn_jvp_fwd_split runs the last query
+ * tiles of these sizes in pieces of their keys (0: it would not; at most
+ * about 70 MB).
+ */
+int dmad_attn_fwd_split_bytes(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk,
+                              int64_t Dv, size_t* bytes);
+
+/*
+ * dmad_attn_jvp_fwd with a second scratch buffer (256-byte aligned). Query
+ * tiles that do not fill a round over the chip are cut along their keys; the
+ * pieces' fp32 results go to split_ws and are combined, in a fixed order, by
+ * a second kernel. With split_ws null or smaller than
+ * dmad_attn_fwd_split_bytes it is dmad_attn_jvp_fwd.
+ */
+int dmad_attn_jvp_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv,
+                            const void* q, const void* k, const void* v, const void* tq, const void* tk,
+                            const void* tv, const int64_t q_strides[4], const int64_t k_strides[4],
+                            const int64_t v_strides[4], void* o, void* to, const int64_t o_strides[4], float* lse,
+                            float* mu, float sm_scale, void* workspace, size_t workspace_bytes, void* split_ws,
+                            size_t split_bytes, void* stream);
+
+/*
  * Block-sparse forward (+JVP): replaces the `_attn_fwd_magi` launch of
  * _attention.forward with a MagiMask (flash_attention_jvp_triton.py:502-531,
  * kernel :242-409). The tables are the MagiMask fields

@@ -1,0 +1,93 @@
+"""Launches whose last work items run in pieces (csrc/split.h).
+
+Each case takes sizes whose plan splits and compares the split call with the same call
+without room for its partials (every tile whole): both against the float64 oracle, the split
+one no further from it than 1.1x the whole one plus 1e-5 (the pieces are combined in fp32;
+what is left is the rounding of P~ against another running maximum). A call must also repeat
+bit for bit.
+"""
+import pytest
+import torch
+
+from oracle import attention as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _draw(dev, seed, B, H, Lq, Lk, D, dtype):
+    g = torch.Generator().manual_seed(seed)
+
+    def r(L, std=1.0):
+        return (torch.randn((B, L, H, D), generator=g, dtype=torch.float64) * std).to(dtype).to(dev).transpose(1, 2)
+
+    return r(Lq), r(Lk), r(Lk), r(Lq, 0.1), r(Lk, 0.1), r(Lk, 0.1)
+
+
+def _no_worse(name, split, whole, ref):
+    e, f = orc.rel_l2(split.cpu(), ref), orc.rel_l2(whole.cpu(), ref)
+    print(f"  {name} split {e:.2e} whole {f:.2e}", flush=True)
+    assert e <= 1.1 * f + 1e-5, (name, e, f)
+
+
+FWD = [
+    # mode, B, H, Lq, Lk, D
+    ("jvp", 1, 2, 999, 999, 128),     # 16 tiles alone on the chip
+    ("jvp", 1, 2, 999, 999, 64),
+    ("jvp", 1, 1, 130, 545, 128),     # 18 steps, the last one key; a partial query tile
+    ("jvp", 2, 1, 257, 2100, 64),
+    ("q", 1, 2, 700, 2047, 128),      # key range of the two-workgroups-per-CU kernel
+    ("q", 1, 1, 300, 4100, 128),
+    ("q", 1, 2, 300, 1000, 64),
+    ("plain", 1, 2, 1000, 1100, 128),
+    ("plain", 1, 2, 333, 1500, 64),
+    ("plain", 1, 1, 1, 3000, 128),    # one query
+    ("jvp", 1, 9, 3700, 2500, 128),   # 261 tiles: a full round, then five tiles in pieces
+    ("plain", 1, 21, 3200, 1100, 128),  # 525 tiles: a full round of two per CU, then 13
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mode,B,H,Lq,Lk,D", FWD)
+def test_split_forward(gpu, monkeypatch, mode, B, H, Lq, Lk, D, dtype):
+    from dmad_amd import _native as nat
+    from dmad_amd.jvp_attention import jvp_attention_forward
+
+    print(f"case split fwd {mode} {B} {H} {Lq} {Lk} {D} {dtype}", flush=True)
+    code = nat.dtype_code(dtype)
+    nmode = {"plain": nat.DMAD_FWD_PLAIN, "jvp": nat.DMAD_FWD_JVP, "q": nat.DMAD_FWD_JVP_KV_TANGENT_ZERO}[mode]
+    q, k, v, tq, tk, tv = _draw(gpu, Lq + Lk + D, B, H, Lq, Lk, D, dtype)
+    args = (q, k, v) + ((None,) * 3 if mode == "plain" else (tq, None, None) if mode == "q" else (tq, tk, tv))
+    assert nat.fwd_split_bytes(code, nmode, B, H, Lq, Lk, D, D) > 0
+    got = jvp_attention_forward(*args, D ** -0.5)
+    again = jvp_attention_forward(*args, D ** -0.5)
+    monkeypatch.setattr(nat, "fwd_split_bytes", lambda *a: 0)
+    whole = jvp_attention_forward(*args, D ** -0.5)
+    torch.cuda.synchronize()
+    for a, b in zip(got, again):
+        assert a is b is None or torch.equal(a, b)
+    heads = [0, H - 1] if H > 3 else list(range(H))
+    xs = [t[:, heads].cpu().double() for t in (q, k, v, tq, tk if mode == "jvp" else torch.zeros_like(k),
+                                               tv if mode == "jvp" else torch.zeros_like(v))]
+    ref = orc.jvp_closed_form(*xs)
+    for name, a, b, r in zip(("o", "to", "lse", "mu"), got, whole, ref):
+        if a is not None:
+            _no_worse(name, a[:, heads], b[:, heads], r)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_split_forward_with_masked_pieces(gpu, D):
+    """Keys that all score -inf in the last pieces (a -inf feature in K, as a caller's padding
+    mask): they weigh nothing, and every row is what the other keys give."""
+    from dmad_amd import _native as nat
+    from dmad_amd.jvp_attention import jvp_attention_forward
+
+    B, H, Lq, Lk, live = 1, 2, 200, 2000, 700
+    assert nat.fwd_split_bytes(nat.DMAD_BF16, nat.DMAD_FWD_PLAIN, B, H, Lq, Lk, D, D) > 0
+    q, k, v, *_ = _draw(gpu, 3, B, H, Lq, Lk, D, torch.bfloat16)
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    k[:, :, live:, 0] = -float("inf")
+    o, _, lse, _ = jvp_attention_forward(q, k, v, None, None, None, D ** -0.5)
+    ro, rlse = orc.math_attention(q.cpu().double(), k[:, :, :live].cpu().double(), v[:, :, :live].cpu().double(), D ** -0.5)
+    assert orc.rel_l2(o.cpu(), ro) <= 1e-2
+    assert float((lse.cpu().double() - rlse).abs().max()) <= 2e-3
