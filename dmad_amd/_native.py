@@ -98,6 +98,12 @@ SIGNATURES = {
                                  _P, _P, _I64P, _P, _P, _P, _P, _I64P,
                                  _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
                                  _F, _P, _SZ, _P]),
+    "dmad_attn_bwd_split_bytes": (_INT, [_INT, _INT, _INT, _I64, _I64, _I64, _I64, _I64, _SZP]),
+    "dmad_attn_jvp_bwd_split": (_INT, [_INT, _I64, _I64, _I64, _I64, _I64,
+                                       _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
+                                       _P, _P, _I64P, _P, _P, _P, _P, _I64P,
+                                       _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
+                                       _F, _P, _SZ, _P, _SZ, _P]),
     "dmad_attn_jvp_bwd_noalloc": (_INT, [_INT, _I64, _I64, _I64, _I64, _I64,
                                          _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
                                          _P, _P, _I64P, _P, _P, _P, _P, _I64P,
@@ -193,6 +199,15 @@ def fwd_split_bytes(dtype: int, mode: int, B: int, H: int, Lq: int, Lk: int, Dqk
     their keys (0: it runs every tile whole)."""
     n = ctypes.c_size_t(0)
     check(lib().dmad_attn_fwd_split_bytes(dtype, mode, B, H, Lq, Lk, Dqk, Dv, ctypes.byref(n)))
+    return int(n.value)
+
+
+@functools.lru_cache(maxsize=1024)
+def bwd_split_bytes(dtype: int, full: bool, tangent_grads: bool, B: int, H: int, Lq: int, Lk: int, D: int) -> int:
+    """Bytes of fp32 partials with which a backward splits its passes' last tiles (0: it runs
+    every tile whole)."""
+    n = ctypes.c_size_t(0)
+    check(lib().dmad_attn_bwd_split_bytes(dtype, int(full), int(tangent_grads), B, H, Lq, Lk, D, ctypes.byref(n)))
     return int(n.value)
 
 

@@ -70,6 +70,7 @@ struct BwdParams {
   void* sc;
   int64_t sc_slice;
   int bh0;
+  SplitParams sp;  // split launches of the row-reading key passes (split.h)
 };
 
 // Layout of the score gradients a key pass stores for the query pass to read
@@ -798,7 +799,9 @@ enum KvScMode : int {
 // wave's two 1 KiB chunks of a tile ride in the ring stage with the Q and dO
 // rows (a lane's 16 bytes land where it reads them), V is not read, and a step
 // runs 8 S MFMAs and 16 update MFMAs instead of 32.
-template <typename T, int D, int SCM = kScNone>
+// SPLIT: the last work items of the grid run in pieces of the queries (split.h),
+// each writing its dK, dV accumulators as partials.
+template <typename T, int D, int SCM = kScNone, bool SPLIT = false>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kv_tr_kernel(BwdParams p) {
   using C = KvTrCfg<D, kKvTrBmq>;
   constexpr int BMQ = C::BMQ, NQB = C::NQB, KS = C::KS, DB = C::DB, CR = C::CR, ROWB = C::ROWB;
@@ -819,12 +822,21 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kv_tr_kernel(Bw
   const int col = lane & 31, half = lane >> 5;
 
   const int nkt = (p.Lk + C::BK - 1) / C::BK;
-  const int work = work_item(p.xcd_order);  // block order (common.h)
+  const int nqt_all = p.LQP / BMQ;
+  int work, qt0 = 0, nqt = nqt_all, part_slot = -1;  // query tiles [qt0, qt0 + nqt) are this workgroup's
+  if constexpr (SPLIT) {
+    const SplitWork w = split_work(p.sp, p.xcd_order, nqt_all);
+    if (w.item < 0) return;
+    work = w.item;
+    qt0 = w.beg;
+    nqt = w.end - w.beg;
+    if (w.piece >= 0) part_slot = w.slot;
+  } else {
+    work = work_item(p.xcd_order);  // block order (common.h)
+  }
   const int slice = work / nkt, kt = work - slice * nkt;
   const int bh = (SCM != kScNone ? p.bh0 : 0) + slice;
   const int b = bh / p.H, h = bh - b * p.H;
-  const int nqt = p.LQP / BMQ;
-
   const int key = kt * C::BK + wave * 32 + col;
 
   // ---- stored score gradients (STORE: dS written; LOAD: tensor 1 of a full
@@ -836,6 +848,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kv_tr_kernel(Bw
   const uint32_t sc_lo0 = ScLayout::lane_off(col, half, 0), sc_lo1 = ScLayout::lane_off(col, half, 1);
   const bool sc_tail = (kt + 1) * C::BK > p.Lk;  // keys at or beyond Lk in this workgroup
   auto store_chunk = [&](int qt, int u, i32x4_t v) {
+    qt += qt0;
     if (sc_tail && key >= p.Lk) v = i32x4_t{0, 0, 0, 0};
     const __amdgpu_buffer_rsrc_t rs =
         make_rsrc(sc_base + (int64_t)(qt >> 2) * sc_strip, (uint32_t)(sc_strip - ScLayout::STRIP_PAD));
@@ -888,11 +901,12 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kv_tr_kernel(Bw
     else if constexpr (k == 2) return (lds_char_t*)stg2;
     else return (lds_char_t*)stg3;
   };
-  // request li (0 <= li < LOADS) of tile qt into stage st; tiles at or beyond
-  // the end read zeros or in-range rows into a stage nobody reads again (the
+  // request li (0 <= li < LOADS) of this workgroup's tile qt into stage st; tiles at
+  // or beyond the end read zeros or in-range rows into a stage nobody reads again (the
   // loaded dS chunks of such tiles are the last tile's again: a strip beyond the
   // slice does not exist)
   auto issue_load = [&](lds_char_t* st, int qt, int li) {
+    qt += qt0;
     if (li < 2 * RPW) {
       const int jj = li >> 1, i = wave + jj * C::NW;
       if (li & 1) buf_load16_lds(rdo, st + C::OFF_DO + i * 1024, roff_do[jj], (uint32_t)qt * do_step);
@@ -900,7 +914,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kv_tr_kernel(Bw
     } else if (li == 2 * RPW) {
       if (st_lane) buf_load16_lds(rst, st + C::OFF_ST, lane * 16, (uint32_t)qt * C::STAT_BYTES);
     } else if constexpr (LOAD) {
-      const int u = li - 2 * RPW - 1, qc = qt < nqt ? qt : nqt - 1;
+      const int u = li - 2 * RPW - 1, qc = qt < nqt_all ? qt : nqt_all - 1;
       const __amdgpu_buffer_rsrc_t rs =
           make_rsrc(sc_base + (int64_t)(qc >> 2) * sc_strip, (uint32_t)(sc_strip - ScLayout::STRIP_PAD));
       buf_load16_lds(rs, st + OFF_DS + wave * 2 * ScLayout::CHUNK + u * ScLayout::CHUNK, u ? sc_lo1 : sc_lo0,
@@ -1145,6 +1159,9 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kv_tr_kernel(Bw
     f32x16_t un_s[NQB], un_p[NQB];
 #pragma unroll
     for (int m = NMA; m < NS; ++m) mfma_slot(m, load_op(s_cur, s_cur, m), un_s, un_p, pb, dsb);
+    // the last dK, dV MFMAs finish before their AGPRs are read: here, ahead of the
+    // copies to VGPRs the compiler makes where the paths through the last steps meet
+    if constexpr (kAccAgpr) mfma_acc_drain(dkacc, dvacc);
   };
 
   if (nqt > 0) {
@@ -1181,7 +1198,22 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kv_tr_kernel(Bw
     else last_step(IC<3>{}, sb, pbb, cb_p, cb_d);
     wait_vmem();  // no requests beyond the last tile stay in flight
   }
-  if constexpr (kAccAgpr) mfma_acc_drain();  // the last dK, dV MFMAs have finished before their AGPRs are read
+
+  if constexpr (SPLIT) {
+    if (part_slot >= 0) {
+      constexpr int TILE = split_tile_floats<D>();
+      float* const tile = p.sp.part + ((int64_t)part_slot * C::NW + wave) * 2 * TILE;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          split_put<D>(tile, lane, d, jj, f32x4_t{dkacc[d][4 * jj], dkacc[d][4 * jj + 1], dkacc[d][4 * jj + 2], dkacc[d][4 * jj + 3]});
+          split_put<D>(tile + TILE, lane, d, jj, f32x4_t{dvacc[d][4 * jj], dvacc[d][4 * jj + 1], dvacc[d][4 * jj + 2], dvacc[d][4 * jj + 3]});
+        }
+      }
+      return;
+    }
+  }
 
   // ---- store dK = s (dK^T)^T, dV = (dV^T)^T for this lane's key
   if (key < p.Lk) {

@@ -52,6 +52,7 @@ struct DqParams {
   int64_t sc_slice;
   int sc_nkb;
   int bh0;
+  SplitParams sp;  // split launches of the row-reading query passes (split.h)
 };
 
 template <int D, int MODE>
@@ -563,7 +564,9 @@ struct DqTrCfg {
 // D = 64 fits three waves per SIMD (168 VGPRs, 32 KiB of LDS per workgroup):
 // the third wave hides more of the 6 VALU instructions per MFMA (1% faster at
 // B=4, H=32, L=16384 than two waves at 172 VGPRs, with bitwise equal dQ).
-template <typename T, int D>
+// SPLIT: the last work items run in pieces of the keys (split.h), each writing
+// its dQ accumulators as partials.
+template <typename T, int D, bool SPLIT = false>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 1) void attn_bwd_dq_tr_kernel(DqParams p) {
   using C = DqTrCfg<D>;
   constexpr int BN = C::BN, KS = C::KS, DB = C::DB, CR = C::CR, ROWB = C::ROWB;
@@ -578,10 +581,19 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 1) void attn_bwd_dq_tr_kernel(Dq
   const int col = lane & 31, half = lane >> 5;
 
   const int nqt = (p.Lq + C::BM - 1) / C::BM;
-  const int work = work_item(p.xcd_order);  // block order (common.h)
+  int work, kt0 = 0, ntiles = (p.Lk + BN - 1) / BN, part_slot = -1;  // key tiles [kt0, kt0 + ntiles) are this workgroup's
+  if constexpr (SPLIT) {
+    const SplitWork w = split_work(p.sp, p.xcd_order, ntiles);
+    if (w.item < 0) return;
+    work = w.item;
+    kt0 = w.beg;
+    ntiles = w.end - w.beg;
+    if (w.piece >= 0) part_slot = w.slot;
+  } else {
+    work = work_item(p.xcd_order);  // block order (common.h)
+  }
   const int bh = work / nqt, qt = work - bh * nqt;
   const int b = bh / p.H, h = bh - b * p.H;
-  const int ntiles = (p.Lk + BN - 1) / BN;
 
   // ---- this lane's query: Q, dO rows (B operands) and statistics
   const int query = qt * C::BM + wave * 32 + col;
@@ -639,6 +651,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 1) void attn_bwd_dq_tr_kernel(Dq
   // request li (0 <= li < C::LOADS) of tile kt into stage st; tiles at or beyond
   // the end read zeros or in-range rows into a stage nobody reads again
   auto issue_load = [&](lds_char_t* st, int kt, int li) {
+    kt += kt0;
     const int jj = li >> 1, i = wave + jj * C::NW;
     if (li & 1) buf_load16_lds(rv, st + C::OFF_V + i * 1024, roff_v[jj], (uint32_t)kt * v_step);
     else buf_load16_lds(rk, st + C::OFF_K + i * 1024, roff_k[jj], (uint32_t)kt * k_step);
@@ -794,6 +807,19 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 1) void attn_bwd_dq_tr_kernel(Dq
     else if (rest == 3) last_step(IC<2>{}, sa, pa);
     else last_step(IC<3>{}, sb, pbb);
     wait_vmem();  // no requests beyond the last tile stay in flight
+  }
+
+  if constexpr (SPLIT) {
+    if (part_slot >= 0) {
+      float* const tile = p.sp.part + ((int64_t)part_slot * C::NW + wave) * split_tile_floats<D>();
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+          split_put<D>(tile, lane, d, jj, f32x4_t{acc[d][4 * jj], acc[d][4 * jj + 1], acc[d][4 * jj + 2], acc[d][4 * jj + 3]});
+      }
+      return;
+    }
   }
 
   // ---- dQ = s (dQ^T)^T: lane holds query col, rows d = 32 db + 8 jj + 4 half + (0..3)

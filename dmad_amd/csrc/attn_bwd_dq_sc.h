@@ -50,7 +50,9 @@ struct DqScCfg {
   static_assert((NSTAGE - 1) * LOADS < 64, "vmcnt is a 6-bit field");
 };
 
-template <typename T, int NT>
+// SPLIT: the last work items run in pieces of the keys (split.h), each writing
+// its dQ (and dQd) accumulators as partials.
+template <typename T, int NT, bool SPLIT = false>
 __global__ __launch_bounds__(512, 1) void attn_bwd_dq_sc_kernel(DqParams p) {
   using C = DqScCfg<NT>;
   constexpr int D = C::D, BN = C::BN, DB = C::DB, CR = C::CR, ROWB = C::ROWB, NSTAGE = C::NSTAGE;
@@ -69,11 +71,21 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dq_sc_kernel(DqParams p) {
 
   const int nqb = (p.Lq + C::BQ - 1) / C::BQ;
   const int npair = (nqb + 1) / 2;
-  const int work = work_item(p.xcd_order);  // block order (common.h)
+  const int nsteps_all = (p.Lk + BN - 1) / BN;
+  int work, j0 = 0, nsteps = nsteps_all, part_slot = -1;  // steps [j0, j0 + nsteps) are this workgroup's
+  if constexpr (SPLIT) {
+    const SplitWork w = split_work(p.sp, p.xcd_order, nsteps_all);
+    if (w.item < 0) return;
+    work = w.item;
+    j0 = w.beg;
+    nsteps = w.end - w.beg;
+    if (w.piece >= 0) part_slot = w.slot;
+  } else {
+    work = work_item(p.xcd_order);  // block order (common.h)
+  }
   const int slice = work / npair, qbp = work - slice * npair;
   const int bh = p.bh0 + slice;
   const int b = bh / p.H, h = bh - b * p.H;
-  const int nsteps = (p.Lk + BN - 1) / BN;
   const int qb = 2 * qbp + blk;  // this wave's query block (qb == nqb: none; its reads repeat block nqb - 1)
   const int query = qb * C::BQ + tile * 32 + col;
 
@@ -95,7 +107,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dq_sc_kernel(DqParams p) {
   // stage st: rows of K [and Kd] (1 KiB each), then the pieces of block 0 and
   // block 1 (steps past the end repeat the last one)
   auto issue_req = [&](lds_char_t* st, int jj, int i) {
-    jj = jj < nsteps ? jj : nsteps - 1;
+    jj = (SPLIT ? j0 : 0) + (jj < nsteps ? jj : nsteps - 1);
     if (i < NT * C::NRI) {
       const int t = i / C::NRI, r = i % C::NRI;
       const int pch = r * 64 + lane;
@@ -219,6 +231,25 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dq_sc_kernel(DqParams p) {
       if (j + 2 < nsteps) step(IC<2>{}, j + 2);
     }
     wait_vmem();  // no requests stay in flight
+  }
+
+  if constexpr (SPLIT) {
+    if (part_slot >= 0) {
+      constexpr int TILE = split_tile_floats<D>();
+      float* const tl = p.sp.part + ((int64_t)part_slot * C::NW + wave) * NT * TILE;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          split_put<D>(tl, lane, d, jj, f32x4_t{acc[d][4 * jj], acc[d][4 * jj + 1], acc[d][4 * jj + 2], acc[d][4 * jj + 3]});
+          if constexpr (NT == 2) {
+            if (p.dtq != nullptr)
+              split_put<D>(tl + TILE, lane, d, jj, f32x4_t{tacc[d][4 * jj], tacc[d][4 * jj + 1], tacc[d][4 * jj + 2], tacc[d][4 * jj + 3]});
+          }
+        }
+      }
+      return;
+    }
   }
 
   // ---- dQ = s (dQ^T)^T [, dQd = s (dQd^T)^T]: lane holds query col, d = 32 db + 8 jj + 4 half + 0..3

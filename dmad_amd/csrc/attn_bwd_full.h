@@ -84,7 +84,8 @@ __device__ __forceinline__ FullVals full_values(float s, float sd_raw, float dpd
 // barrier's vmcnt(LOADS) stays exact whatever order stores and loads complete
 // in: a request of tile j + 2 still in flight means all LOADS requests of tile
 // j + 3 are too.
-template <typename T, int D, bool STORE = false>
+// SPLIT: as attn_bwd_kv_tr_kernel.
+template <typename T, int D, bool STORE = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void attn_bwd_kv_full_kernel(BwdParams p) {
   using C = KvFullCfg<D>;
   constexpr int BMQ = C::BMQ, KS = C::KS, DB = C::DB, CR = C::CR, ROWB = C::ROWB;
@@ -99,11 +100,20 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kv_full_kernel(BwdParams p) {
   const int col = lane & 31, half = lane >> 5;
 
   const int nkt = (p.Lk + C::BK - 1) / C::BK;
-  const int work = work_item(p.xcd_order);  // block order (common.h)
+  int work, qt0 = 0, nqt = p.LQP / BMQ, part_slot = -1;  // query tiles [qt0, qt0 + nqt) are this workgroup's
+  if constexpr (SPLIT) {
+    const SplitWork w = split_work(p.sp, p.xcd_order, nqt);
+    if (w.item < 0) return;
+    work = w.item;
+    qt0 = w.beg;
+    nqt = w.end - w.beg;
+    if (w.piece >= 0) part_slot = w.slot;
+  } else {
+    work = work_item(p.xcd_order);  // block order (common.h)
+  }
   const int slice = work / nkt, kt = work - slice * nkt;
   const int bh = (STORE ? p.bh0 : 0) + slice;
   const int b = bh / p.H, h = bh - b * p.H;
-  const int nqt = p.LQP / BMQ;
   const int key = kt * C::BK + wave * 32 + col;
 
   // ---- score-gradient stores (STORE): this wave's key block of the slice's strips
@@ -114,6 +124,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kv_full_kernel(BwdParams p) {
   const bool sc_tail = (kt + 1) * C::BK > p.Lk;  // keys at or beyond Lk in this workgroup
   // chunk u of tensor t (0: dS, 1: dSd) of tile qt
   auto store_chunk = [&](int qt, int t, int u, i32x4_t v) {
+    qt += qt0;
     if (sc_tail && key >= p.Lk) v = i32x4_t{0, 0, 0, 0};
     const __amdgpu_buffer_rsrc_t rs =
         make_rsrc(sc_base + (int64_t)(qt >> 2) * sc_strip, (uint32_t)(sc_strip - ScLayout::STRIP_PAD));
@@ -180,6 +191,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kv_full_kernel(BwdParams p) {
   // request li (0 <= li < LOADS) of query tile qt into stage st: row pieces of
   // Q, dO, Qd, dOd, then the statistics; tiles at or beyond the end read zeros
   auto issue_load = [&](lds_char_t* st, int qt, int li) {
+    qt += qt0;
     if (li < 4 * RPW) {
       const int t = li % 4, jj = li / 4, i = wave + jj * C::NW;
       const uint32_t qs = (uint32_t)qt * q_step, ds = (uint32_t)qt * do_step;
@@ -375,6 +387,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kv_full_kernel(BwdParams p) {
     Scores un;
 #pragma unroll
     for (int o = NOPA; o < NOP; ++o) mfma_op(o, load_op(s_cur, s_cur, o), un, pk);
+    mfma_acc_drain(dkacc, dvacc);  // before any path reads the AGPRs (as attn_bwd_kv_tr_kernel)
   };
 
   if (nqt > 0) {
@@ -409,7 +422,22 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kv_full_kernel(BwdParams p) {
     else last_step(IC<3>{}, sb);
     wait_vmem();  // no requests beyond the last tile stay in flight
   }
-  mfma_acc_drain();  // the last dK, dV MFMAs have finished before their AGPRs are read
+
+  if constexpr (SPLIT) {
+    if (part_slot >= 0) {
+      constexpr int TILE = split_tile_floats<D>();
+      float* const tile = p.sp.part + ((int64_t)part_slot * C::NW + wave) * 2 * TILE;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          split_put<D>(tile, lane, d, jj, f32x4_t{dkacc[d][4 * jj], dkacc[d][4 * jj + 1], dkacc[d][4 * jj + 2], dkacc[d][4 * jj + 3]});
+          split_put<D>(tile + TILE, lane, d, jj, f32x4_t{dvacc[d][4 * jj], dvacc[d][4 * jj + 1], dvacc[d][4 * jj + 2], dvacc[d][4 * jj + 3]});
+        }
+      }
+      return;
+    }
+  }
 
   // ---- store dK = s (dK^T)^T, dV = (dV^T)^T for this lane's key
   if (key < p.Lk) {
@@ -693,6 +721,8 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_full_kernel(DqParams p) {
     Scores un;
 #pragma unroll
     for (int o = NOPA; o < NOP; ++o) mfma_op(o, load_op(s_cur, s_cur, o), un, pk);
+    if constexpr (TG) mfma_acc_drain(acc, tacc);  // before any path reads the AGPRs
+    else mfma_acc_drain(acc);
   };
 
   if (ntiles > 0) {
@@ -727,7 +757,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_full_kernel(DqParams p) {
     else last_step(IC<3>{}, sb);
     wait_vmem();  // no requests beyond the last tile stay in flight
   }
-  mfma_acc_drain();
 
   // ---- dQ = s (dQ^T)^T [, dQd = s (dQd^T)^T]: lane holds query col, d = 32 db + 8 jj + 4 half + 0..3
   if (query < p.Lq) {

@@ -660,7 +660,7 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
     else last_step(IC<5>{}, i + 5, sb, tb);
   }
   wait_vmem();  // no requests beyond the last tile stay in flight
-  if constexpr (kAccAgpr) mfma_acc_drain();
+  if constexpr (kAccAgpr) mfma_acc_drain(oacc, cacc);
 
   // ---- epilogue: lane (query col, half) holds d = 32 db + 8 jj + 4 half + (0..3)
   const float l = l_i + other_half(l_i);

@@ -37,4 +37,16 @@ DqLaunchFn dq_tr_select<Elt, 256>() {
   return &dq_tr_launch<Elt, 256>;
 }
 
+// split launches
+template <typename T, int D>
+static hipError_t dq_split_launch(const DqParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_bwd_dq_tr_kernel<T, D, true>), dim3(grid), dim3(256), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_dq_sum<T, D, DqTrCfg<D>::NW, 1>(p, s);
+}
+template <>
+DqLaunchFn dq_split_select<Elt>(int d) {
+  return d == 64 ? &dq_split_launch<Elt, 64> : d == 128 ? &dq_split_launch<Elt, 128> : nullptr;
+}
+
 }  // namespace dmad

@@ -59,4 +59,26 @@ DqLaunchFn dq_full_select<Elt>(bool tangent_grads) {
   return tangent_grads ? &dq_full_launch<Elt, true> : &dq_full_launch<Elt, false>;
 }
 
+// split launches
+template <typename T, bool STORE>
+static hipError_t kv_full_split_launch(const BwdParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_bwd_kv_full_kernel<T, 128, STORE, true>), dim3(grid), dim3(256), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_kv_sum<T, 128>(p, s);
+}
+template <>
+BwdLaunchFn kv_full_split_select<Elt>(bool store) {
+  return store ? &kv_full_split_launch<Elt, true> : &kv_full_split_launch<Elt, false>;
+}
+template <typename T>
+static hipError_t dq_sc2_split_launch(const DqParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_bwd_dq_sc_kernel<T, 2, true>), dim3(grid), dim3(DqScCfg<2>::NW * 64), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_dq_sum<T, 128, DqScCfg<2>::NW, 2>(p, s);
+}
+template <>
+DqLaunchFn dq_sc_split_select<Elt>(bool full) {
+  return full ? &dq_sc2_split_launch<Elt> : dq_sc_split_dout_only<Elt>();
+}
+
 }  // namespace dmad

@@ -62,4 +62,31 @@ BwdLaunchFn kv_sc_tangent<Elt>() {
   return &kv_ld_launch<Elt>;
 }
 
+// split launches
+template <typename T, int D, int SCM>
+static hipError_t kv_split_launch(const BwdParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_bwd_kv_tr_kernel<T, D, SCM, true>), dim3(grid), dim3(256), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_kv_sum<T, D>(p, s);
+}
+template <>
+BwdLaunchFn kv_split_select<Elt>(int d, int scm) {
+  if (d == 64) return scm == kScNone ? &kv_split_launch<Elt, 64, kScNone> : nullptr;
+  if (d != 128) return nullptr;
+  return scm == kScNone    ? &kv_split_launch<Elt, 128, kScNone>
+         : scm == kScStore ? &kv_split_launch<Elt, 128, kScStore>
+                           : &kv_split_launch<Elt, 128, kScLoad>;
+}
+// NT = 1; the full derivative's (NT = 2) in bwd_full_inst.hip
+template <typename T>
+static hipError_t dq_sc1_split_launch(const DqParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_bwd_dq_sc_kernel<T, 1, true>), dim3(grid), dim3(DqScCfg<1>::NW * 64), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_dq_sum<T, 128, DqScCfg<1>::NW, 1>(p, s);
+}
+template <>
+DqLaunchFn dq_sc_split_dout_only<Elt>() {
+  return &dq_sc1_split_launch<Elt>;
+}
+
 }  // namespace dmad

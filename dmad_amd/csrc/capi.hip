@@ -505,6 +505,79 @@ BwdPlan plan_bwd_ws(int dtype, bool full, bool tgrad, int64_t B, int64_t H, int6
   return pl;
 }
 
+// Split launches of the backward's row-reading passes (split.h): the last key
+// tiles run in pieces of the queries, the last query tiles (pairs of tiles on
+// stored gradients) in pieces of the keys. The cut depends on the sizes alone and
+// is the same whether scores are stored or recomputed and however many (b, h)
+// slices a launch pair takes, so dK and dV keep not depending on the workspace.
+struct BwdSplit {
+  dmad::SplitPlan kv;    // main key pass
+  dmad::SplitPlan kv_t;  // tangent key pass
+  dmad::SplitPlan dq;    // recomputing query pass (dO only; with tangent gradients of 64-wide heads theirs)
+  dmad::SplitPlan dq_sc; // query pass on stored gradients
+  int64_t bytes = 0;     // the largest of their partials (one after the other in a call)
+};
+
+BwdSplit plan_bwd_split(int dtype, bool full, bool tgrad, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D) {
+  BwdSplit r;
+  if ((dtype != DMAD_BF16 && dtype != DMAD_F16) || (D != 64 && D != 128)) return r;
+  const int64_t BH = B * H, nkt = (Lk + 127) / 128, nqt = (Lq + 127) / 128, qsteps = round_up(Lq, 64) / 32,
+                ksteps = (Lk + 31) / 32;
+  const int tile = (int)D * 32 * 4;  // bytes of one wave's accumulator tile
+  // Costs for plan_split; measured (bf16 unless said, H=12, the second number split,
+  // the sum kernel included): 6240 tokens, 76 of 588 key tiles and 44 of 300 query
+  // pairs in pieces: full key pass 1280 -> 1170 us, its query pass 492 -> 380,
+  // tangent key pass 429 -> 381; 10920 tokens, dO only: key pass 1534 -> 1480, query
+  // pass 644 -> 540; 999 tokens of two fp16 64-wide heads: 23.2 -> 15.5 and 18.5 ->
+  // 11.7. Where whole tiles already keep more than half of the chip busy for a few
+  // dozen steps the partials cost more than the split saves (1560 tokens, key pass:
+  // 47-50 us whole, 54-65 split), and the costs keep them whole.
+  const dmad::SplitCost kv = D == 128 ? dmad::SplitCost{1, 0.85f, 0.f, 10.f, 8 * tile}
+                                      : dmad::SplitCost{2, 0.5f, 0.8f, 7.f, 8 * tile};
+  const dmad::SplitCost kv_full{1, 2.0f, 0.f, 12.f, 8 * tile};
+  const dmad::SplitCost dq = D == 128 ? dmad::SplitCost{2, 0.6f, 0.8f, 8.f, 4 * tile}
+                                      : dmad::SplitCost{3, 0.35f, 0.6f, 5.f, 4 * tile};
+  const dmad::SplitCost dq_sc{1, full ? 1.2f : 0.6f, 0.f, 8.f, (full ? 16 : 8) * tile};
+  if (!full || D == 128) r.kv = dmad::plan_split(BH * nkt, qsteps, full ? kv_full : kv);
+  if (tgrad) r.kv_t = dmad::plan_split(BH * nkt, qsteps, kv);
+  if (!full || (tgrad && D == 64)) r.dq = dmad::plan_split(BH * nqt, ksteps, dq);
+  if (D == 128) r.dq_sc = dmad::plan_split(BH * ((nqt + 1) / 2), ksteps, dq_sc);
+  for (const dmad::SplitPlan* p : {&r.kv, &r.kv_t, &r.dq, &r.dq_sc}) r.bytes = p->bytes > r.bytes ? p->bytes : r.bytes;
+  return r;
+}
+
+// The part of a split that falls in work items [first, first + items) of the call
+// (one launch pair's slices); rest == 0 where it holds none of the split items.
+dmad::SplitParams split_of_launch(const dmad::SplitPlan& pl, int64_t first, int64_t items, void* part) {
+  if (pl.rest == 0 || part == nullptr) return dmad::SplitParams{};
+  const int64_t w = pl.whole - first, whole = w < 0 ? 0 : w < items ? w : items;
+  return dmad::SplitParams{(int)whole, (int)(items - whole), pl.n, pl.len, (float*)part};
+}
+
+dmad::BwdLaunchFn pick_kv_split(int dtype, int64_t d, bool full, int scm) {
+  if (dtype == DMAD_BF16)
+    return full ? dmad::kv_full_split_select<__bf16>(scm == dmad::kScStore) : dmad::kv_split_select<__bf16>((int)d, scm);
+  if (dtype == DMAD_F16)
+    return full ? dmad::kv_full_split_select<_Float16>(scm == dmad::kScStore) : dmad::kv_split_select<_Float16>((int)d, scm);
+  return nullptr;
+}
+
+dmad::DqLaunchFn pick_dq_split(int dtype, int64_t d, bool full, bool stored) {
+  if (dtype == DMAD_BF16) return stored ? dmad::dq_sc_split_select<__bf16>(full) : dmad::dq_split_select<__bf16>((int)d);
+  if (dtype == DMAD_F16) return stored ? dmad::dq_sc_split_select<_Float16>(full) : dmad::dq_split_select<_Float16>((int)d);
+  return nullptr;
+}
+
+// One pass over work items [first, first + items) of a call: split where the plan
+// says so and there is room for the partials, else `whole` on the ordinary grid.
+template <typename Params, typename Fn>
+hipError_t launch_pass(Params p, Fn whole, Fn split, const dmad::SplitPlan& pl, int64_t first, int64_t items,
+                       void* part, hipStream_t s) {
+  p.sp = split != nullptr ? split_of_launch(pl, first, items, part) : dmad::SplitParams{};
+  if (p.sp.rest == 0) return whole(p, (int)items, s);
+  return split(p, (int)dmad::split_grid(p.sp.whole, p.sp.rest, p.sp.n), s);
+}
+
 // Shared body of the dense and block-sparse forwards (mg == nullptr: dense).
 int fwd_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv, const void* q,
              const void* k, const void* v, const void* tq, const void* tk, const void* tv, const int64_t q_strides[4],
@@ -688,7 +761,8 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
              const int64_t o_strides[4], const float* lse, const float* mu, const void* dout, const void* dto,
              const int64_t do_strides[4], void* dq, void* dk, void* dv, void* dtq, void* dtk, void* dtv,
              const int64_t dq_strides[4], const int64_t dk_strides[4], const int64_t dv_strides[4], float sm_scale,
-             void* workspace, size_t workspace_bytes, void* stream, bool use_scratch) {
+             void* workspace, size_t workspace_bytes, void* split_ws, size_t split_bytes, void* stream,
+             bool use_scratch) {
   if (dtype != DMAD_BF16 && dtype != DMAD_F16 && dtype != DMAD_F32)
     return fail(DMAD_ERR_UNSUPPORTED, "unsupported dtype code %d", dtype);
   if (B < 0 || H < 0 || Lq < 0 || Lk < 0) return fail(DMAD_ERR_INVALID, "negative size");
@@ -746,6 +820,10 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
     return fail(DMAD_ERR_WORKSPACE, "workspace needs %lld bytes, got %lld", (long long)w.total, (long long)workspace_bytes);
   // workspace beyond the minimum holds stored score gradients (128-wide bf16/fp16 heads)
   const int64_t sc = use_scratch ? 0 : score_slices(dtype, full, B, H, Lq, Lk, D, w.total, (int64_t)workspace_bytes);
+  if (((uintptr_t)split_ws & 255) != 0) return fail(DMAD_ERR_INVALID, "the split workspace must be 256-byte aligned");
+  BwdSplit split;
+  if (split_ws != nullptr) split = plan_bwd_split(dtype, full, tgrad, B, H, Lq, Lk, D);
+  void* const part = split.bytes > 0 && (int64_t)split_bytes >= split.bytes ? split_ws : nullptr;
   if (((uintptr_t)workspace & 255) != 0) return fail(DMAD_ERR_INVALID, "workspace must be 256-byte aligned");
   const int64_t dp = D < 32 ? 32 : D, lqp = round_up(Lq, 64), lkp = round_up(Lk, kLkAlign), BH = B * H;
   if (dp * lqp * 2 >= kMaxHeadBytes || dp * lkp * 2 >= kMaxHeadBytes) return fail(DMAD_ERR_UNSUPPORTED, "sequence too long");
@@ -947,31 +1025,37 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
     pt.dv = dtv;
     pq.sc_nkb = (int)(4 * nkt);
     pq.xcd_order = nqw < dmad::kHeadMajorMinTiles;
+    const dmad::BwdLaunchFn fs_sp = pick_kv_split(dtype, D, full, dmad::kScStore);
+    const dmad::BwdLaunchFn fts_sp = pick_kv_split(dtype, D, false, dmad::kScLoad);
+    const dmad::DqLaunchFn fqs_sp = pick_dq_split(dtype, D, full, true);
     int ev = 0;
     for (int64_t bh0 = 0; bh0 < BH; bh0 += sc) {
       const int64_t n = BH - bh0 < sc ? BH - bh0 : sc;
       p.bh0 = pq.bh0 = pt.bh0 = (int)bh0;
       mark(ev, false, s);
-      if ((e = fs(p, (int)(n * nkt), s)) != hipSuccess) return fail(DMAD_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
+      if ((e = launch_pass(p, fs, fs_sp, split.kv, bh0 * nkt, n * nkt, part, s)) != hipSuccess) return fail(DMAD_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
       mark(ev++, true, s);
       mark(ev, false, s);
-      if ((e = fqs(pq, (int)(n * nqw), s)) != hipSuccess)
+      if ((e = launch_pass(pq, fqs, fqs_sp, split.dq_sc, bh0 * nqw, n * nqw, part, s)) != hipSuccess)
         return fail(DMAD_ERR_HIP, "backward dq launch: %s", hipGetErrorString(e));
       mark(ev++, true, s);
       if (tgrad) {
         mark(ev, false, s);
-        if ((e = fts(pt, (int)(n * nkt), s)) != hipSuccess)
+        if ((e = launch_pass(pt, fts, fts_sp, split.kv_t, bh0 * nkt, n * nkt, part, s)) != hipSuccess)
           return fail(DMAD_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
         mark(ev++, true, s);
       }
     }
     return ok();
   }
+  const dmad::BwdLaunchFn fn_sp = pick_kv_split(dtype, D, full, dmad::kScNone);
+  const dmad::BwdLaunchFn fa_sp = pick_kv_split(dtype, D, false, dmad::kScNone);
+  const dmad::DqLaunchFn fq_sp = pick_dq_split(dtype, D, full, false);
   mark(0, false, s);
-  if ((e = fn(p, (int)plan.grid_kv, s)) != hipSuccess) return fail(DMAD_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
+  if ((e = launch_pass(p, fn, fn_sp, split.kv, 0, plan.grid_kv, part, s)) != hipSuccess) return fail(DMAD_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
   mark(0, true, s);
   mark(1, false, s);
-  if (plan.grid_dq > 0 && (e = fq(pq, (int)plan.grid_dq, s)) != hipSuccess)
+  if (plan.grid_dq > 0 && (e = launch_pass(pq, fq, full ? nullptr : fq_sp, split.dq, 0, plan.grid_dq, part, s)) != hipSuccess)
     return fail(DMAD_ERR_HIP, "backward dq launch: %s", hipGetErrorString(e));
   mark(1, true, s);
   if (tgrad) {
@@ -984,7 +1068,7 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
     pt.dk = dtk;
     pt.dv = dtv;
     mark(2, false, s);
-    if ((e = fn_a(pt, (int)plan.grid_kv, s)) != hipSuccess)
+    if ((e = launch_pass(pt, fn_a, fa_sp, split.kv_t, 0, plan.grid_kv, part, s)) != hipSuccess)
       return fail(DMAD_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
     mark(2, true, s);
     dmad::DqParams pqt = pq;
@@ -994,7 +1078,7 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
     pqt.dq = dtq;
     if (fq_a != nullptr) {
       mark(3, false, s);
-      if (plan.grid_dq > 0 && (e = fq_a(pqt, (int)plan.grid_dq, s)) != hipSuccess)
+      if (plan.grid_dq > 0 && (e = launch_pass(pqt, fq_a, fq_sp, split.dq, 0, plan.grid_dq, part, s)) != hipSuccess)
         return fail(DMAD_ERR_HIP, "backward dq launch: %s", hipGetErrorString(e));
       mark(3, true, s);
     }
@@ -1172,7 +1256,30 @@ int dmad_attn_jvp_bwd(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, i
                       void* stream) {
   return bwd_impl(dtype, B, H, Lq, Lk, D, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to, o_strides, lse,
                   mu, dout, dto, do_strides, dq, dk, dv, dtq, dtk, dtv, dq_strides, dk_strides, dv_strides, sm_scale,
-                  workspace, workspace_bytes, stream, false);
+                  workspace, workspace_bytes, nullptr, 0, stream, false);
+}
+
+int dmad_attn_bwd_split_bytes(int dtype, int full, int tangent_grads, int64_t B, int64_t H, int64_t Lq, int64_t Lk,
+                              int64_t D, size_t* bytes) {
+  if (bytes == nullptr) return fail(DMAD_ERR_INVALID, "bytes: null pointer");
+  if ((full != 0 && full != 1) || (tangent_grads != 0 && tangent_grads != 1))
+    return fail(DMAD_ERR_INVALID, "full and tangent_grads must be 0 or 1");
+  if (B < 0 || H < 0 || Lq < 0 || Lk < 0 || !head_dim_ok(D)) return fail(DMAD_ERR_INVALID, "bad sizes");
+  *bytes = (size_t)plan_bwd_split(dtype, full != 0, tangent_grads != 0, B, H, Lq, Lk, D).bytes;
+  return ok();
+}
+
+int dmad_attn_jvp_bwd_split(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D, const void* q,
+                            const void* k, const void* v, const void* tq, const void* tk, const void* tv,
+                            const int64_t q_strides[4], const int64_t k_strides[4], const int64_t v_strides[4],
+                            const void* o, const void* to, const int64_t o_strides[4], const float* lse,
+                            const float* mu, const void* dout, const void* dto, const int64_t do_strides[4], void* dq,
+                            void* dk, void* dv, void* dtq, void* dtk, void* dtv, const int64_t dq_strides[4],
+                            const int64_t dk_strides[4], const int64_t dv_strides[4], float sm_scale, void* workspace,
+                            size_t workspace_bytes, void* split_ws, size_t split_bytes, void* stream) {
+  return bwd_impl(dtype, B, H, Lq, Lk, D, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to, o_strides, lse,
+                  mu, dout, dto, do_strides, dq, dk, dv, dtq, dtk, dtv, dq_strides, dk_strides, dv_strides, sm_scale,
+                  workspace, workspace_bytes, split_ws, split_bytes, stream, false);
 }
 
 int dmad_attn_jvp_bwd_noalloc(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D, const void* q,
@@ -1185,7 +1292,7 @@ int dmad_attn_jvp_bwd_noalloc(int dtype, int64_t B, int64_t H, int64_t Lq, int64
                               float sm_scale, void* stream) {
   return bwd_impl(dtype, B, H, Lq, Lk, D, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to, o_strides, lse,
                   mu, dout, dto, do_strides, dq, dk, dv, dtq, dtk, dtv, dq_strides, dk_strides, dv_strides, sm_scale,
-                  nullptr, 0, stream, true);
+                  nullptr, 0, nullptr, 0, stream, true);
 }
 
 int dmad_rmsnorm_rope_jvp(int dtype, int64_t rows, int64_t L, int64_t H, int64_t D, const void* y, const void* ty,

@@ -144,8 +144,18 @@ __device__ __forceinline__ void mfma32_acc(f32x16_t& c, i32x4_t a, i32x4_t b, _F
   asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 // 24 wait states: more than an in-flight 32x32x16 MFMA needs before its result
-// is read.
-__device__ __forceinline__ void mfma_acc_drain() { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory"); }
+// is read. The accumulators are re-defined after the wait: nothing else keeps the
+// compiler from copying them out of their AGPRs before it (it hoists copies that
+// two branches after the wait share).
+template <int... N>
+__device__ __forceinline__ void mfma_acc_drain(f32x16_t (&... acc)[N]) {
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+  auto redefine = [](auto& a) {
+#pragma unroll
+    for (auto& block : a) asm volatile("" : "+a"(block));
+  };
+  (redefine(acc), ...);
+}
 
 // 16x16x32 layouts: A (16 x 32): lane l holds row l%16, k = 8*(l/16) + e;
 // B (32 x 16): lane l holds col l%16, k = 8*(l/16) + e;

@@ -131,6 +131,49 @@ DqLaunchFn dq_sc_select(bool full);
 template <> DqLaunchFn dq_sc_select<__bf16>(bool);
 template <> DqLaunchFn dq_sc_select<_Float16>(bool);
 
+// The row-reading passes with their last work items in pieces, each followed by
+// the kernel that sums the pieces (BwdParams::sp, DqParams::sp; split.h): the key
+// pass of d-wide heads by what it does with score gradients (d = 64: kScNone), the
+// full key pass (store: kScStore), the recomputing query pass and the query pass
+// on stored gradients.
+template <typename T>
+BwdLaunchFn kv_split_select(int d, int scm);
+template <> BwdLaunchFn kv_split_select<__bf16>(int, int);
+template <> BwdLaunchFn kv_split_select<_Float16>(int, int);
+template <typename T>
+BwdLaunchFn kv_full_split_select(bool store);
+template <> BwdLaunchFn kv_full_split_select<__bf16>(bool);
+template <> BwdLaunchFn kv_full_split_select<_Float16>(bool);
+template <typename T>
+DqLaunchFn dq_split_select(int d);
+template <> DqLaunchFn dq_split_select<__bf16>(int);
+template <> DqLaunchFn dq_split_select<_Float16>(int);
+template <typename T>
+DqLaunchFn dq_sc_split_dout_only();
+template <> DqLaunchFn dq_sc_split_dout_only<__bf16>();
+template <> DqLaunchFn dq_sc_split_dout_only<_Float16>();
+template <typename T>
+DqLaunchFn dq_sc_split_select(bool full);
+template <> DqLaunchFn dq_sc_split_select<__bf16>(bool);
+template <> DqLaunchFn dq_sc_split_select<_Float16>(bool);
+
+// Sums the pieces of a split key pass (dK, dV) or query pass (dQ [, dQd]).
+template <typename T, int D>
+hipError_t launch_kv_sum(const BwdParams& p, hipStream_t s) {
+  SplitSumParams c{p.sp, {p.dk, p.dv}, {p.dk_sb, p.dv_sb}, {p.dk_sh, p.dv_sh}, {p.dk_sl, p.dv_sl}, {p.scale, 1.f},
+                   p.H, p.Lk, (p.Lk + 127) / 128, p.bh0};
+  hipLaunchKernelGGL((split_sum_kernel<T, D, 4, 2>), dim3(4 * p.sp.rest), dim3(256), 0, s, c);
+  return hipGetLastError();
+}
+template <typename T, int D, int WAVES, int NT>
+hipError_t launch_dq_sum(const DqParams& p, hipStream_t s) {
+  constexpr int BM = 32 * WAVES;
+  SplitSumParams c{p.sp, {p.dq, NT == 2 ? p.dtq : nullptr}, {p.dq_sb, p.dq_sb}, {p.dq_sh, p.dq_sh}, {p.dq_sl, p.dq_sl},
+                   {p.scale, p.scale}, p.H, p.Lq, (p.Lq + BM - 1) / BM, p.bh0};
+  hipLaunchKernelGGL((split_sum_kernel<T, D, WAVES, NT>), dim3(WAVES * p.sp.rest), dim3(256), 0, s, c);
+  return hipGetLastError();
+}
+
 // Query tile of the dK/dV kernel, which fixes the layout of the backward
 // statistics (the full-derivative kernel always uses 32-query tiles).
 inline int bwd_bmq(int d, int mode) {

@@ -263,4 +263,65 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdCombineParams p) {
   }
 }
 
+// ---------------------------------------------------------------- backward
+// Partial block of a backward pass: [waves][tensors][32 x D] accumulator tiles,
+// unscaled. The passes' pieces add up without weights.
+struct SplitSumParams {
+  SplitParams sp;
+  void* out[2];  // dK, dV or dQ, dQd; out[1] may be null (its tiles are then not read)
+  int64_t sb[2], sh[2], sl[2];
+  float scale[2];
+  int H, L;      // rows of an output's head
+  int tiles;     // work items per head
+  int bh0;       // head of work item 0
+};
+
+// One workgroup per wave tile (32 rows) of a split item, four pieces' loads in
+// flight at a time (as fwd_combine_kernel). WAVES waves per work item, NT tiles
+// per wave.
+template <typename T, int D, int WAVES, int NT>
+__global__ __launch_bounds__(256) void split_sum_kernel(SplitSumParams p) {
+  constexpr int TILE = split_tile_floats<D>(), FLOATS = WAVES * NT * TILE;
+  const int item = (int)blockIdx.x / WAVES, wave = (int)blockIdx.x - item * WAVES;
+  const int lane = lane_id(), col = lane & 31, half = lane >> 5, grp = threadIdx.x >> 6;
+  const int work = p.sp.whole + item, slice = work / p.tiles, tile_no = work - slice * p.tiles;
+  const int bh = p.bh0 + slice, b = bh / p.H, h = bh - b * p.H;
+  const int row = (tile_no * WAVES + wave) * 32 + col;
+  const float* part = p.sp.part + (int64_t)item * p.sp.n * FLOATS + wave * NT * TILE;
+  constexpr int U = 4, NG = D / 32;
+  const int n = p.sp.n;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (p.out[t] == nullptr) continue;
+    f32x4_t acc[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) acc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < n; i += U) {
+      f32x4_t v[U][NG];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float* tile = part + (int64_t)min(i + u, n - 1) * FLOATS + t * TILE;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) v[u][g] = split_get<D>(tile, lane, 4 * g + grp);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (i + u >= n) break;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) acc[g] += v[u][g];
+      }
+    }
+    if (row < p.L) {
+      char* out = (char*)p.out[t] + (b * p.sb[t] + h * p.sh[t] + (int64_t)row * p.sl[t]) * 2;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const f32x4_t a = acc[g] * p.scale[t];
+        *(u32x2_t*)(out + (32 * g + 8 * grp + 4 * half) * 2) =
+            u32x2_t{Elem<T>::pack2(a[0], a[1]), Elem<T>::pack2(a[2], a[3])};
+      }
+    }
+  }
+}
+
 }  // namespace dmad

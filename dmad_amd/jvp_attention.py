@@ -467,8 +467,9 @@ def jvp_attention_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto, sm_sc
     lib = nat.lib()
     ws_mode = (2 if tgrads else 1) if full else 0
     ws_ptr, ws_size, ws = _backward_workspace(code, ws_mode, B, H, Lq, Lk, D, q.device)
+    sp_ptr, sp_size, sp = _split_workspace(nat.bwd_split_bytes(code, full, tgrads, B, H, Lq, Lk, D), q.device)
     nat.check(
-        lib.dmad_attn_jvp_bwd(
+        lib.dmad_attn_jvp_bwd_split(
             code, B, H, Lq, Lk, D,
             nat.ptr(q), nat.ptr(k), nat.ptr(v), nat.ptr(tq), nat.ptr(tk), nat.ptr(tv),
             nat.strides4(q), nat.strides4(k), nat.strides4(v),
@@ -476,7 +477,7 @@ def jvp_attention_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto, sm_sc
             nat.ptr(dout), nat.ptr(dto), nat.strides4(dout),
             nat.ptr(dq), nat.ptr(dk), nat.ptr(dv), nat.ptr(dtq), nat.ptr(dtk), nat.ptr(dtv),
             nat.strides4(dq), nat.strides4(dk), nat.strides4(dv),
-            float(sm_scale), ws_ptr, ws_size, nat.stream_ptr(q.device),
+            float(sm_scale), ws_ptr, ws_size, sp_ptr, sp_size, nat.stream_ptr(q.device),
         )
     )
     return dq, dk, dv, dtq, dtk, dtv

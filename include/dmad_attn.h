@@ -175,6 +175,24 @@ int dmad_attn_jvp_bwd(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, i
                       const int64_t dv_strides[4], float sm_scale, void* workspace, size_t workspace_bytes,
                       void* stream);
 
+/*
+ * dmad_attn_jvp_bwd with a second scratch buffer for partials, as
+ * dmad_attn_jvp_fwd_split: the passes of 64- and 128-wide bf16/fp16 heads run
+ * the key (query) tiles that do not fill a round over the chip in pieces. With
+ * split_ws null or smaller than dmad_attn_bwd_split_bytes it is
+ * dmad_attn_jvp_bwd. full and tangent_grads as for dmad_attn_bwd_plan.
+ */
+int dmad_attn_bwd_split_bytes(int dtype, int full, int tangent_grads, int64_t B, int64_t H, int64_t Lq, int64_t Lk,
+                              int64_t D, size_t* bytes);
+int dmad_attn_jvp_bwd_split(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D, const void* q,
+                            const void* k, const void* v, const void* tq, const void* tk, const void* tv,
+                            const int64_t q_strides[4], const int64_t k_strides[4], const int64_t v_strides[4],
+                            const void* o, const void* to, const int64_t o_strides[4], const float* lse,
+                            const float* mu, const void* dout, const void* dto, const int64_t do_strides[4], void* dq,
+                            void* dk, void* dv, void* dtq, void* dtk, void* dtv, const int64_t dq_strides[4],
+                            const int64_t dk_strides[4], const int64_t dv_strides[4], float sm_scale, void* workspace,
+                            size_t workspace_bytes, void* split_ws, size_t split_bytes, void* stream);
+
 /* Size of the static device scratch of dmad_attn_jvp_bwd_noalloc (64 MiB). */
 #define DMAD_BWD_SCRATCH_BYTES ((size_t)64 << 20)
 

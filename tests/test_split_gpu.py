@@ -91,3 +91,53 @@ def test_split_forward_with_masked_pieces(gpu, D):
     ro, rlse = orc.math_attention(q.cpu().double(), k[:, :, :live].cpu().double(), v[:, :, :live].cpu().double(), D ** -0.5)
     assert orc.rel_l2(o.cpu(), ro) <= 1e-2
     assert float((lse.cpu().double() - rlse).abs().max()) <= 2e-3
+
+
+BWD = [
+    # B, H, Lq, Lk, D, full derivative with tangent gradients
+    (1, 2, 999, 999, 64, False),
+    (1, 2, 999, 999, 128, False),    # recomputing query pass
+    (1, 2, 2111, 2111, 128, False),  # stored score gradients
+    (1, 2, 700, 905, 128, True),
+    (1, 2, 900, 700, 64, True),      # the tangent passes of 64-wide heads
+    (2, 1, 130, 3000, 128, False),   # few query tiles, a partial one
+    (1, 1, 3000, 33, 64, False),     # one key tile, 94 query steps
+    (1, 9, 3700, 3700, 128, False),  # 261 key tiles: one after the full round, in pieces
+    (1, 9, 3700, 3700, 128, True),
+    (1, 27, 2500, 2500, 64, False),  # 540 key tiles of two per CU; 540 query tiles of three
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Lq,Lk,D,full", BWD)
+def test_split_backward(gpu, monkeypatch, B, H, Lq, Lk, D, full, dtype):
+    """The tiles' P and dS do not change, only the order in which fp32 sums add up, so a split
+    gradient differs from the whole one by output roundings that fall the other way."""
+    from dmad_amd import _native as nat
+    from dmad_amd.jvp_attention import jvp_attention_backward, jvp_attention_forward
+
+    print(f"case split bwd {B} {H} {Lq} {Lk} {D} full={full} {dtype}", flush=True)
+    code = nat.dtype_code(dtype)
+    assert nat.bwd_split_bytes(code, full, full, B, H, Lq, Lk, D) > 0
+    q, k, v, tq, tk, tv = _draw(gpu, Lq + Lk + D, B, H, Lq, Lk, D, dtype)
+    do, _, _, dto, _, _ = _draw(gpu, 1, B, H, Lq, Lk, D, dtype)
+    s = D ** -0.5
+    o, to, lse, mu = jvp_attention_forward(q, k, v, tq, tk, tv, s)
+
+    def backward():
+        return jvp_attention_backward(q, k, v, tq, tk, tv, o, to, lse, mu, do, dto if full else None, s, full)
+
+    got, again = backward(), backward()
+    monkeypatch.setattr(nat, "bwd_split_bytes", lambda *a: 0)
+    whole = backward()
+    torch.cuda.synchronize()
+    names = ("dq", "dk", "dv", "dtq", "dtk", "dtv")
+    for name, a, b, w in zip(names, got, again, whole):
+        assert a is b is w is None or (torch.equal(a, b) and
+                                       orc.rel_l2(a.cpu(), w.cpu()) <= (2 ** -9 if dtype == torch.bfloat16 else 2 ** -12)), name
+    if H > 2:
+        return
+    xs = [t.cpu().double() for t in (q, k, v, tq, tk, tv, do, dto)]
+    ref = orc.grads_full(*xs) if full else orc.grads_dout_only(*xs[:3], xs[6])
+    for name, a, w, r in zip(names, got, whole, ref):
+        _no_worse(name, a, w, r)
