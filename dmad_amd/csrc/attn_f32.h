@@ -99,7 +99,9 @@ struct F32FwdCfg {
   static_assert(LDS_FLOATS * 4 <= 160 * 1024, "tile exceeds LDS");
 };
 
-template <int DQK, int DV, int MODE, bool MAGI>
+// SPLIT (dense, Dqk = Dv up to 128): the last query tiles run in pieces of their
+// keys (split.h).
+template <int DQK, int DV, int MODE, bool MAGI, bool SPLIT = false>
 __global__ __launch_bounds__(f32_fwd_wide(MODE, DQK) ? 256 : 512) void attn_f32_fwd_kernel(FwdParams p) {
   using C = F32FwdCfg<DQK, DV, MODE, MAGI>;
   static_assert(C::NT == (f32_fwd_wide(MODE, DQK) ? 256 : 512), "launch bounds match the workgroup");
@@ -119,7 +121,19 @@ __global__ __launch_bounds__(f32_fwd_wide(MODE, DQK) ? 256 : 512) void attn_f32_
   int bh, row0, chunk, ntiles;
   int q_lo = 0, q_hi = p.Lq;  // rows this workgroup stores
   MagiCursor cm{0, 0, 0, 0, 0};
-  if constexpr (MAGI) {
+  int kt0 = 0, part_slot = -1;  // SPLIT: first key tile and partial block of this piece
+  static_assert(!SPLIT || (!MAGI && C::NCH == 1 && C::BM == 128), "split launches: dense, all of V in one workgroup");
+  if constexpr (SPLIT) {
+    const int nqt = (p.Lq + C::BM - 1) / C::BM;
+    const SplitWork w = split_work(p.sp, p.xcd_order, (p.Lk + BN - 1) / BN);
+    if (w.item < 0) return;
+    chunk = 0;
+    bh = w.item / nqt;
+    row0 = (w.item - bh * nqt) * C::BM;
+    kt0 = w.beg;
+    ntiles = w.end - w.beg;
+    if (w.piece >= 0) part_slot = w.slot;
+  } else if constexpr (MAGI) {
     const int work = xcd_remap(blockIdx.x, p.T * p.B * p.H * C::NCH * C::HALVES);
     chunk = work % C::NCH;
     const int half = (work / C::NCH) % C::HALVES;  // 64-row half of the task (one-wave-per-SIMD form)
@@ -244,15 +258,16 @@ __global__ __launch_bounds__(f32_fwd_wide(MODE, DQK) ? 256 : 512) void attn_f32_
     oacc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     cacc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  float m_i = -__builtin_inff(), l_i = 0.f, r_i = 0.f;
+  // (a piece starts from a finite maximum: attn_fwd32_kernel)
+  float m_i = SPLIT ? -3.0e38f : -__builtin_inff(), l_i = 0.f, r_i = 0.f;
 
   auto fetch = [&](int start) {
     fetch_k(start);
     fetch_v(start);
   };
-  if constexpr (C::PREFETCH) fetch(MAGI ? ci.start : 0);
+  if constexpr (C::PREFETCH) fetch(MAGI ? ci.start : kt0 * BN);
   for (int kt = 0; kt < ntiles; ++kt) {
-    const int start = MAGI ? cm.start : kt * BN;
+    const int start = MAGI ? cm.start : (kt0 + kt) * BN;
     __syncthreads();  // every wave is done with the previous tile
     if constexpr (C::WIDE && !C::PREFETCH) {  // K rows, then V: half the staging registers live at once
       fetch_k(start);
@@ -266,7 +281,7 @@ __global__ __launch_bounds__(f32_fwd_wide(MODE, DQK) ? 256 : 512) void attn_f32_
     }
     if constexpr (MAGI) ci.next(p, BN);
     if constexpr (C::PREFETCH) {
-      if (kt + 1 < ntiles) fetch(MAGI ? ci.start : (kt + 1) * BN);
+      if (kt + 1 < ntiles) fetch(MAGI ? ci.start : (kt0 + kt + 1) * BN);
     }
     __syncthreads();
 
@@ -371,6 +386,25 @@ __global__ __launch_bounds__(f32_fwd_wide(MODE, DQK) ? 256 : 512) void attn_f32_
   const float inv_l = 1.0f / l;
   float mu = 0.f;
   if constexpr (C::JVP) mu = quad_sum(r_i) * inv_l;
+  if constexpr (SPLIT) {
+    if (part_slot >= 0) {
+      using P = FwdPart<DV, C::JVP, 16>;
+      float* const part = p.sp.part + (int64_t)part_slot * P::FLOATS;
+      float* const tile = part + wave * P::NT * P::TILE;
+      const float keep_l = l == 0.f ? 0.f : inv_l;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        *(f32x4_t*)(tile + (d * 64 + lane) * 4) = oacc[d] * keep_l;
+        if constexpr (C::JVP) *(f32x4_t*)(tile + P::TILE + (d * 64 + lane) * 4) = cacc[d] * keep_l;
+      }
+      if (g == 0) {
+        float* const st = part + P::STATS + wave * 32 + col;
+        st[0] = m_i + __builtin_log2f(l);
+        if constexpr (C::JVP) st[16] = l == 0.f ? 0.f : mu;
+      }
+      return;
+    }
+  }
   const int64_t obase = b * p.o_sb + h * p.o_sh;
   const uint32_t o_bytes = (uint32_t)(((int64_t)(p.Lq - 1) * p.o_sl + DV) * 4);
   const __amdgpu_buffer_rsrc_t ro = make_rsrc((float*)p.o + obase, o_bytes);

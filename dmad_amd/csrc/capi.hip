@@ -281,6 +281,16 @@ dmad::SplitCost fwd_split_cost(int mode, int64_t D) {
   return {4, 0.3f, 0.6f, 6.f, dmad::FwdPart<64, false>::FLOATS * 4};
 }
 
+// The same for attn_f32_fwd_kernel, whose step is bound by its fp32 MFMAs: 6.5 us
+// for the 32 keys of a 64-wide JVP step, so few tiles split down to single steps.
+// Measured (JVP, the second number split): two 64-wide heads of 256 tokens 53.8 ->
+// 16.0 us (eight pieces), of 999 tokens 200 -> 33.4 us; 12 heads of 1560 tokens, 156
+// tiles in two uneven pieces each, 310 -> 219 us at 64 and 598 -> 417 us at 128 wide.
+dmad::SplitCost f32_fwd_split_cost(int mode, int64_t D) {
+  const bool jvp = mode != DMAD_FWD_PLAIN;
+  return {1, (jvp ? 0.1f : 0.035f) * (float)D, 0.f, 6.f, (int)((128 * D * (jvp ? 2 : 1) + 256) * 4)};
+}
+
 // The split of a dense forward's last query tiles over their keys. Both JVP
 // modes split alike (with the full JVP's costs), so that O does not depend on
 // whether Kd = Vd = 0 was stated; they split no key range of 512 or fewer, which
@@ -291,12 +301,23 @@ dmad::SplitPlan plan_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_
   const int64_t items = (Lq + 127) / 128 * B * H, steps = (Lk + 31) / 32;
   dmad::SplitPlan none;
   none.whole = none.grid = items;
-  if (dtype == DMAD_F32 || !dmad::fwd32_supported((int)Dqk, (int)Dv)) return none;
+  if (dtype == DMAD_F32)
+    return dmad::f32_fwd_splits((int)Dqk, (int)Dv) ? dmad::plan_split(items, steps, f32_fwd_split_cost(mode, Dqk)) : none;
+  if (!dmad::fwd32_supported((int)Dqk, (int)Dv)) return none;
   if (mode != DMAD_FWD_PLAIN && (steps <= 16 || (steps <= kX2MaxKeyTiles && items >= dmad::kSplitCus))) return none;
   return dmad::plan_split(items, steps, fwd_split_cost(mode, Dqk));
 }
 
 dmad::FwdLaunchFn pick_fwd_split(int dtype, int64_t d, int mode) {
+  if (dtype == DMAD_F32) {
+    switch (d) {
+      case 16: return dmad::f32_fwd_split_select<16>(mode);
+      case 32: return dmad::f32_fwd_split_select<32>(mode);
+      case 64: return dmad::f32_fwd_split_select<64>(mode);
+      case 128: return dmad::f32_fwd_split_select<128>(mode);
+    }
+    return nullptr;
+  }
   if (dtype == DMAD_BF16) return dmad::fwd32_split_select<__bf16>(mode, (int)d);
   if (dtype == DMAD_F16) return dmad::fwd32_split_select<_Float16>(mode, (int)d);
   return nullptr;

@@ -28,6 +28,29 @@ static hipError_t f32_fwd_launch(const FwdParams& p, int grid, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int D, int MODE>
+static hipError_t f32_fwd_split_launch(const FwdParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_f32_fwd_kernel<D, D, MODE, false, true>), dim3(grid),
+                     dim3(F32FwdCfg<D, D, MODE, false>::NT), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  FwdCombineParams c{p.sp, p.o, p.to, p.lse, p.mu, p.o_sb, p.o_sh, p.o_sl, p.H, p.Lq};
+  hipLaunchKernelGGL((fwd_combine_kernel<float, D, MODE != kFwdPlain, 16>), dim3(8 * p.sp.rest), dim3(256), 0, s, c);
+  return hipGetLastError();
+}
+
+template <>
+FwdLaunchFn f32_fwd_split_select<DMAD_D>(int mode) {
+  if constexpr (f32_fwd_splits(DMAD_D, DMAD_D)) {
+    switch (mode) {
+      case kFwdPlain: return &f32_fwd_split_launch<DMAD_D, kFwdPlain>;
+      case kFwdJvp: return &f32_fwd_split_launch<DMAD_D, kFwdJvp>;
+      case kFwdJvpQOnly: return &f32_fwd_split_launch<DMAD_D, kFwdJvpQOnly>;
+    }
+  }
+  return nullptr;
+}
+
 template <int DQK, int DV>
 static FwdLaunchFn f32_fwd_mode(int mode, bool magi) {
   if (magi) {

@@ -220,6 +220,16 @@ template <> FwdLaunchFn f32_fwd_select<32>(int, int, bool);
 template <> FwdLaunchFn f32_fwd_select<64>(int, int, bool);
 template <> FwdLaunchFn f32_fwd_select<128>(int, int, bool);
 template <> FwdLaunchFn f32_fwd_select<256>(int, int, bool);
+// The same with the last query tiles in pieces of their keys, and the combining
+// kernel (FwdParams::sp), for the head dims of f32_fwd_splits.
+constexpr bool f32_fwd_splits(int dqk, int dv) { return dqk == dv && dqk <= 128; }
+template <int DQK>
+FwdLaunchFn f32_fwd_split_select(int mode);
+template <> FwdLaunchFn f32_fwd_split_select<16>(int);
+template <> FwdLaunchFn f32_fwd_split_select<32>(int);
+template <> FwdLaunchFn f32_fwd_split_select<64>(int);
+template <> FwdLaunchFn f32_fwd_split_select<128>(int);
+template <> FwdLaunchFn f32_fwd_split_select<256>(int);
 // V columns per workgroup: 128 in the JVP modes, all of V with 256-wide Q, K
 // (one wave per SIMD, f32_fwd_wide); the plain forward takes up to 256 columns
 // at every Q, K width

@@ -12,6 +12,7 @@
 // What a launch does is decided once per shape on the host (plan_split) from the
 // items, the steps of an item's loop and the costs of the kernel that runs it.
 #pragma once
+#include <type_traits>
 #include "common.h"
 
 namespace dmad {
@@ -64,7 +65,6 @@ template <int D>
 __device__ __forceinline__ void split_put(float* tile, int lane, int d, int jj, f32x4_t v) {
   *(f32x4_t*)(tile + ((4 * d + jj) * 64 + lane) * 4) = v;
 }
-template <int D>
 __device__ __forceinline__ f32x4_t split_get(const float* tile, int lane, int g) {
   return *(const f32x4_t*)(tile + (g * 64 + lane) * 4);
 }
@@ -125,7 +125,7 @@ inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k) {
   const double round = (1. + k.shared * (k.occ - 1)) * k.step * (double)steps + k.fixed;
   const double as_is = split_makespan(k, rest, (double)steps, 0, 0.);
   double best = as_is - 0.05 * (as_is + (double)rounds * round);
-  for (int64_t n = 2; n <= kSplitMaxPieces && 2 * n <= steps; ++n) {
+  for (int64_t n = 2; n <= kSplitMaxPieces && n <= steps; ++n) {
     const double extra = 5. + 2. * (double)(rest * n) * k.part_bytes / 3.3e6;
     const int64_t even = (steps + n - 1) / n;
     // the shorter last piece runs in the slots the n - 1 long ones leave free
@@ -156,15 +156,18 @@ inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k) {
 }
 
 // ---------------------------------------------------------------- forward
-// Partial block of the forward: [4 waves][O (, C)][32 x D], then per wave
-// [lse2, mu][32 rows]. O = O~ / l and C = C~ / l of the piece's keys, lse2 its
-// log2-domain logsumexp.
-template <int D, bool JVP>
+// Partial block of the forward, 128 queries: per wave [O (, C)][ROWS x D], then per
+// wave [lse2, mu][ROWS]. O = O~ / l and C = C~ / l of the piece's keys, lse2 its
+// log2-domain logsumexp. ROWS = 32: tiles as above. ROWS = 16 (fp32 operands): the
+// 16x16 layout (lane: row lane % 16, columns 16 d + 4 (lane / 16) + 0..3), again
+// 16 bytes per lane and d.
+template <int D, bool JVP, int ROWS = 32>
 struct FwdPart {
+  static constexpr int WAVES = 128 / ROWS;
   static constexpr int NT = JVP ? 2 : 1;
-  static constexpr int TILE = split_tile_floats<D>();
-  static constexpr int STATS = 4 * NT * TILE;
-  static constexpr int FLOATS = STATS + 4 * 2 * 32;
+  static constexpr int TILE = ROWS * D;
+  static constexpr int STATS = WAVES * NT * TILE;
+  static constexpr int FLOATS = STATS + WAVES * 2 * ROWS;
 };
 
 struct FwdCombineParams {
@@ -177,30 +180,33 @@ struct FwdCombineParams {
   int H, Lq;
 };
 
-// One workgroup per wave tile (32 queries) of a split item; thread = (lane of the
+// One workgroup per wave tile (ROWS queries) of a split item; thread = (lane of the
 // tile, one of 4 groups of columns). Bound by reading the partials once.
-template <typename T, int D, bool JVP>
+template <typename T, int D, bool JVP, int ROWS = 32>
 __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdCombineParams p) {
-  using P = FwdPart<D, JVP>;
-  const int item = (int)blockIdx.x >> 2, wave = (int)blockIdx.x & 3;
-  const int lane = lane_id(), col = lane & 31, half = lane >> 5, grp = threadIdx.x >> 6;
+  using P = FwdPart<D, JVP, ROWS>;
+  constexpr int GROUPS = ROWS * D / 256;          // 16-byte column groups of a tile's lane
+  constexpr int NG = (GROUPS + 3) / 4;            // ... per thread: groups grp, grp + 4, ...
+  constexpr int U = NG * (JVP ? 2 : 1) > 8 ? 2 : 4;  // pieces in flight
+  const int item = (int)blockIdx.x / P::WAVES, wave = (int)blockIdx.x % P::WAVES;
+  const int lane = lane_id(), col = lane % ROWS, half = lane / ROWS, grp = threadIdx.x >> 6;
+  if (grp >= GROUPS) return;
   const int nqt = (p.Lq + 127) / 128;
   const int work = p.sp.whole + item, bh = work / nqt, qt = work - bh * nqt;
-  const int query = qt * 128 + wave * 32 + col;
+  const int query = qt * 128 + wave * ROWS + col;
   const float* part = p.sp.part + (int64_t)item * p.sp.n * P::FLOATS;
-  const float* st = part + P::STATS + wave * 64 + col;
+  const float* st = part + P::STATS + wave * 2 * ROWS + col;
   // pieces are taken U at a time with all of their loads in flight together (the
   // partials come from other XCDs' workgroups, about a microsecond away); past
   // the last piece the last one is read again and left out
-  constexpr int U = 4, NG = D / 32;  // NG: 16-byte column groups per thread
   const int n = p.sp.n;
   float m = -__builtin_inff();
-  for (int i = 0; i < n; i += 2 * U) {
-    float v[2 * U];
+  for (int i = 0; i < n; i += 8) {
+    float v[8];
 #pragma unroll
-    for (int u = 0; u < 2 * U; ++u) v[u] = st[(int64_t)min(i + u, n - 1) * P::FLOATS];
+    for (int u = 0; u < 8; ++u) v[u] = st[(int64_t)min(i + u, n - 1) * P::FLOATS];
 #pragma unroll
-    for (int u = 0; u < 2 * U; ++u) m = fmaxf(m, v[u]);
+    for (int u = 0; u < 8; ++u) m = fmaxf(m, v[u]);
   }
   float w = 0.f, mu = 0.f;
   f32x4_t o[NG], c[NG];
@@ -212,13 +218,14 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdCombineParams p) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const float* pi = part + (int64_t)min(i + u, n - 1) * P::FLOATS;
-      lse2[u] = pi[P::STATS + wave * 64 + col];
-      if constexpr (JVP) mus[u] = pi[P::STATS + wave * 64 + 32 + col];
+      lse2[u] = pi[P::STATS + wave * 2 * ROWS + col];
+      if constexpr (JVP) mus[u] = pi[P::STATS + wave * 2 * ROWS + ROWS + col];
       const float* tile = pi + wave * P::NT * P::TILE;
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        ov[u][g] = split_get<D>(tile, lane, 4 * g + grp);
-        if constexpr (JVP) cv[u][g] = split_get<D>(tile + P::TILE, lane, 4 * g + grp);
+        const int j = 4 * g + grp < GROUPS ? 4 * g + grp : grp;
+        ov[u][g] = split_get(tile, lane, j);
+        if constexpr (JVP) cv[u][g] = split_get(tile + P::TILE, lane, j);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -245,16 +252,22 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdCombineParams p) {
   const int64_t off = b * p.o_sb + h * p.o_sh + (int64_t)query * p.o_sl;
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    const int dc = 32 * g + 8 * grp + 4 * half;
-    float ov[4], tv[4];
+    if (4 * g + grp >= GROUPS) break;
+    const int dc = (4 * g + grp) * (256 / ROWS) + 4 * half;  // a group is 256 / ROWS columns wide
+    f32x4_t ov, tv;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       ov[e] = o[g][e] * inv;
       tv[e] = c[g][e] * inv - mu * ov[e];
     }
-    *(u32x2_t*)((char*)p.o + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(ov[0], ov[1]), Elem<T>::pack2(ov[2], ov[3])};
-    if constexpr (JVP)
-      *(u32x2_t*)((char*)p.to + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(tv[0], tv[1]), Elem<T>::pack2(tv[2], tv[3])};
+    if constexpr (std::is_same<T, float>::value) {
+      *(f32x4_t*)((float*)p.o + off + dc) = ov;
+      if constexpr (JVP) *(f32x4_t*)((float*)p.to + off + dc) = tv;
+    } else {
+      *(u32x2_t*)((char*)p.o + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(ov[0], ov[1]), Elem<T>::pack2(ov[2], ov[3])};
+      if constexpr (JVP)
+        *(u32x2_t*)((char*)p.to + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(tv[0], tv[1]), Elem<T>::pack2(tv[2], tv[3])};
+    }
   }
   if (half == 0 && grp == 0) {
     const int64_t si = (int64_t)bh * p.Lq + query;
@@ -302,7 +315,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(SplitSumParams p) {
       for (int u = 0; u < U; ++u) {
         const float* tile = part + (int64_t)min(i + u, n - 1) * FLOATS + t * TILE;
 #pragma unroll
-        for (int g = 0; g < NG; ++g) v[u][g] = split_get<D>(tile, lane, 4 * g + grp);
+        for (int g = 0; g < NG; ++g) v[u][g] = split_get(tile, lane, 4 * g + grp);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

@@ -26,7 +26,8 @@ def _draw(dev, seed, B, H, Lq, Lk, D, dtype):
 def _no_worse(name, split, whole, ref):
     e, f = orc.rel_l2(split.cpu(), ref), orc.rel_l2(whole.cpu(), ref)
     print(f"  {name} split {e:.2e} whole {f:.2e}", flush=True)
-    assert e <= 1.1 * f + 1e-5, (name, e, f)
+    # fp32: a few more roundings of 2^-24 each
+    assert e <= 1.1 * f + (4 * 2 ** -24 if split.dtype == whole.dtype == torch.float32 and f < 1e-5 else 1e-5), (name, e, f)
 
 
 FWD = [
@@ -46,8 +47,18 @@ FWD = [
 ]
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("mode,B,H,Lq,Lk,D", FWD)
+FWD_F32 = [
+    ("jvp", 1, 2, 256, 256, 64),   # eight steps, a piece each
+    ("q", 1, 2, 300, 150, 128),
+    ("plain", 1, 1, 100, 2333, 16),
+    ("jvp", 1, 1, 129, 1097, 32),
+    ("plain", 1, 2, 200, 900, 128),
+    ("jvp", 1, 21, 1700, 417, 64),  # 294 tiles: a full round, then 38
+]
+
+
+@pytest.mark.parametrize("mode,B,H,Lq,Lk,D,dtype", [(*c, t) for c in FWD for t in (torch.bfloat16, torch.float16)] +
+                         [(*c, torch.float32) for c in FWD_F32])
 def test_split_forward(gpu, monkeypatch, mode, B, H, Lq, Lk, D, dtype):
     from dmad_amd import _native as nat
     from dmad_amd.jvp_attention import jvp_attention_forward
@@ -74,16 +85,16 @@ def test_split_forward(gpu, monkeypatch, mode, B, H, Lq, Lk, D, dtype):
             _no_worse(name, a[:, heads], b[:, heads], r)
 
 
-@pytest.mark.parametrize("D", [64, 128])
-def test_split_forward_with_masked_pieces(gpu, D):
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.bfloat16), (128, torch.float16), (64, torch.float32)])
+def test_split_forward_with_masked_pieces(gpu, D, dtype):
     """Keys that all score -inf in the last pieces (a -inf feature in K, as a caller's padding
     mask): they weigh nothing, and every row is what the other keys give."""
     from dmad_amd import _native as nat
     from dmad_amd.jvp_attention import jvp_attention_forward
 
     B, H, Lq, Lk, live = 1, 2, 200, 2000, 700
-    assert nat.fwd_split_bytes(nat.DMAD_BF16, nat.DMAD_FWD_PLAIN, B, H, Lq, Lk, D, D) > 0
-    q, k, v, *_ = _draw(gpu, 3, B, H, Lq, Lk, D, torch.bfloat16)
+    assert nat.fwd_split_bytes(nat.dtype_code(dtype), nat.DMAD_FWD_PLAIN, B, H, Lq, Lk, D, D) > 0
+    q, k, v, *_ = _draw(gpu, 3, B, H, Lq, Lk, D, dtype)
     q[..., 0] = 1.0
     k[..., 0] = 0.0
     k[:, :, live:, 0] = -float("inf")
