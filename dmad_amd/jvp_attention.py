@@ -301,9 +301,26 @@ def _pair(x, tx):
     """(primal, tangent) in a layout the kernels read, with equal strides."""
     if tx is None:
         return (x if _kernel_ready(x) else x.contiguous()), None
-    if x.stride() == tx.stride() and _kernel_ready(x) and _kernel_ready(tx):
+    # one layout check serves both where they are laid out alike
+    if x.stride() == tx.stride() and _kernel_ready(x) and (
+            tx.data_ptr() % 16 == 0 if x.dtype == tx.dtype and x.shape == tx.shape else _kernel_ready(tx)):
         return x, tx
     return x.contiguous(), tx.contiguous()
+
+
+_PLAIN_TENSORS = {torch.Tensor, torch.nn.Parameter, type(None)}
+
+
+def _eager_call(*ts) -> bool:
+    """Whether this is an ordinary eager call, which runs the kernels straight from Python:
+    nothing that watches or replaces operators (a compiler, torch.jit tracing, a dispatch or
+    function mode such as selective checkpointing's or make_fx's, a functorch transform,
+    forward-mode AD, a tensor subclass, the profiler) needs to see the registered op. The op
+    costs about 7 us of host time per call beyond the call it wraps (15 us)."""
+    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+                or torch._C._is_torch_function_mode_enabled() or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+                or torch.autograd._profiler_enabled()) and _PLAIN_TENSORS.issuperset(map(type, ts))
 
 
 def _fwd_ws_bytes(dtype, mode, B, H, Lk, Dqk, Dv) -> int:
@@ -483,6 +500,14 @@ def jvp_attention_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto, sm_sc
     return dq, dk, dv, dtq, dtk, dtv
 
 
+def _dout_only_backward(dout, q, k, v, o, lse, sm_scale):
+    """(dQ, dK, dV) inside an autograd backward; the registered op where the gradients are
+    themselves recorded (create_graph), which it refuses to differentiate."""
+    if not torch.is_grad_enabled() and _eager_call(dout, q, k, v, o, lse):
+        return jvp_attention_backward(q, k, v, None, None, None, o, None, lse, None, dout, None, sm_scale, False)[:3]
+    return torch.ops.dmad.flash_attn_bwd(dout, q, k, v, o, lse, sm_scale)
+
+
 class _attention(torch.autograd.Function):
     """
     Arguments:
@@ -531,7 +556,10 @@ class _attention(torch.autograd.Function):
         # an output that does not reach the loss arrives in backward as None
         # (not zeros), so an unused `to` keeps the dO-only kernel
         ctx.set_materialize_grads(False)
-        o, to, lse, mu = torch.ops.dmad.flash_attn_jvp_fwd(q, k, v, tq, tk, tv, float(sm_scale))
+        if _eager_call(q, k, v, tq, tk, tv):
+            o, to, lse, mu = jvp_attention_forward(q, k, v, tq, tk, tv, sm_scale)
+        else:
+            o, to, lse, mu = torch.ops.dmad.flash_attn_jvp_fwd(q, k, v, tq, tk, tv, float(sm_scale))
         if is_grad or tangent_grad:
             if full:
                 ctx.save_for_backward(q, k, v, tq, tk, tv, o, to, lse, mu)
@@ -552,8 +580,7 @@ class _attention(torch.autograd.Function):
             )
             if dout is None:
                 return (None,) * 8
-            dq, dk, dv = torch.ops.dmad.flash_attn_bwd(dout, q, k, v, o, lse, ctx.sm_scale)
-            return dq, dk, dv, None, None, None, None, None
+            return (*_dout_only_backward(dout, q, k, v, o, lse, ctx.sm_scale), None, None, None, None, None)
         q, k, v, tq, tk, tv, o, to, lse, mu = ctx.saved_tensors
         assert q.shape[-1] == k.shape[-1] and k.shape[-1] == v.shape[-1], (
             "Backward not supported with different headdim."
@@ -562,11 +589,16 @@ class _attention(torch.autograd.Function):
             return (None,) * 8
         if dout is None:
             dout = torch.zeros_like(o)
-        dq, dk, dv, dtq, dtk, dtv = torch.ops.dmad.flash_attn_jvp_bwd(
-            q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto, ctx.sm_scale, ctx.tangent_grad
-        )
-        # absent gradients come back from the op as 0-element tensors
-        dtq, dtk, dtv = (None if g.numel() == 0 and x.numel() != 0 else g for g, x in ((dtq, q), (dtk, k), (dtv, v)))
+        if not torch.is_grad_enabled() and _eager_call(q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto):
+            dq, dk, dv, dtq, dtk, dtv = jvp_attention_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto,
+                                                               ctx.sm_scale, ctx.tangent_grad)
+        else:
+            dq, dk, dv, dtq, dtk, dtv = torch.ops.dmad.flash_attn_jvp_bwd(
+                q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto, ctx.sm_scale, ctx.tangent_grad
+            )
+            # absent gradients come back from the op as 0-element tensors
+            dtq, dtk, dtv = (None if g.numel() == 0 and x.numel() != 0 else g
+                             for g, x in ((dtq, q), (dtk, k), (dtv, v)))
         if tk is None:
             dtk = None
         if tv is None:
@@ -659,6 +691,7 @@ def _(dout, q, k, v, o, lse, sm_scale):
 def _fwd_setup_context(ctx, inputs, output):
     q, k, v, sm_scale = inputs
     o, lse = output
+    ctx.set_materialize_grads(False)  # no zeros for the LSE's unused cotangent
     ctx.save_for_backward(q, k, v, o, lse)
     ctx.sm_scale = sm_scale
 
@@ -666,11 +699,27 @@ def _fwd_setup_context(ctx, inputs, output):
 def _fwd_backward(ctx, dout, dlse):
     q, k, v, o, lse = ctx.saved_tensors
     assert q.shape[-1] == v.shape[-1], "Backward not supported with different headdim."
-    dq, dk, dv = torch.ops.dmad.flash_attn_bwd(dout, q, k, v, o, lse, ctx.sm_scale)
-    return dq, dk, dv, None
+    if dout is None:  # only the LSE reached the loss, and its cotangent is not propagated
+        dout = torch.zeros_like(o)
+    return (*_dout_only_backward(dout, q, k, v, o, lse, ctx.sm_scale), None)
 
 
 flash_attn_fwd.register_autograd(_fwd_backward, setup_context=_fwd_setup_context)
+
+
+class _plain_attention(torch.autograd.Function):
+    """O of flash_attn_fwd in an ordinary eager call, with the same backward."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, sm_scale):
+        o, _, lse, _ = jvp_attention_forward(q, k, v, None, None, None, sm_scale)
+        ctx.save_for_backward(q, k, v, o, lse)
+        ctx.sm_scale = sm_scale
+        return o
+
+    @staticmethod
+    def backward(ctx, dout):
+        return _fwd_backward(ctx, dout, None)
 
 
 def plain_attention(q, k, v, sm_scale=None):
@@ -680,4 +729,8 @@ def plain_attention(q, k, v, sm_scale=None):
     assert q.shape[-1] in _HEAD_DIMS and v.shape[-1] in _HEAD_DIMS
     if sm_scale is None:
         sm_scale = q.shape[-1] ** (-0.5)
+    if _eager_call(q, k, v):
+        if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+            return _plain_attention.apply(q, k, v, float(sm_scale))
+        return jvp_attention_forward(q, k, v, None, None, None, sm_scale)[0]
     return torch.ops.dmad.flash_attn_fwd(q, k, v, float(sm_scale))[0]
