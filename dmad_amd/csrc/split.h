@@ -114,7 +114,10 @@ inline double split_makespan(const SplitCost& k, int64_t a, double la, int64_t b
 
 // How to run `items` work items of `steps` steps: in full rounds, then the rest in
 // the pieces that finish soonest by the costs above, where that saves at least a
-// twentieth of the launch. The partials are written and read once, at about
+// twentieth of the launch and 8 us: the second kernel and its scratch cost the host
+// 4-5 us, and calls that short wait for the host (a training call of two 64-wide
+// heads of 999 tokens: 45 us of kernels split, 67 whole, in 200 us of host time,
+// 12 of them for the three splits). The partials are written and read once, at about
 // 3.3 TB/s, by a second kernel that takes 5 us at least (all measured).
 inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k) {
   SplitPlan pl;
@@ -124,7 +127,8 @@ inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k) {
   if (rest == 0 || steps < 4) return pl;
   const double round = (1. + k.shared * (k.occ - 1)) * k.step * (double)steps + k.fixed;
   const double as_is = split_makespan(k, rest, (double)steps, 0, 0.);
-  double best = as_is - 0.05 * (as_is + (double)rounds * round);
+  const double least = 0.05 * (as_is + (double)rounds * round);
+  double best = as_is - (least > 8. ? least : 8.);
   for (int64_t n = 2; n <= kSplitMaxPieces && n <= steps; ++n) {
     const double extra = 5. + 2. * (double)(rest * n) * k.part_bytes / 3.3e6;
     const int64_t even = (steps + n - 1) / n;
