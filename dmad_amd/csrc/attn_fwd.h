@@ -1227,10 +1227,16 @@ __global__ __launch_bounds__(256) void attn_fwd_simple_kernel(FwdParams p) {
 // Transpose X [B,H,L,D] (element strides sb, sh, sl; unit stride in D) ->
 // Y [B*H][DP][LP] contiguous, zero where l >= L or d >= D.
 struct TransposeParams {
-  const void* x;
-  void* y;
-  int64_t sb, sh, sl;
-  int H, L, D, LP, DP;
+  struct Tensor {
+    const void* x;  // [B, H, L, D] with these strides
+    void* y;        // [B*H][DP][LP]
+    int64_t sb, sh, sl;
+    int L, LP;
+  };
+  static constexpr int MAX = 6;
+  Tensor t[MAX];
+  int count;  // tensors to transpose
+  int H, D, DP;
 };
 
 }  // namespace dmad

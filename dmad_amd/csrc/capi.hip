@@ -669,14 +669,14 @@ int fwd_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, 
   // transposed, key-padded copy made here
   const bool need_vt = plan.copies > 0;
   hipError_t e = hipSuccess;
-  dmad::TransposeParams tp{v, ws, v_strides[0], v_strides[1], v_strides[2], (int)H, (int)Lk, (int)Dv, (int)lkp, (int)dvp};
-  if (need_vt) e = dmad::launch_transpose_pad(tp, BH, s);
-  if (e != hipSuccess) return fail(DMAD_ERR_HIP, "transpose launch: %s", hipGetErrorString(e));
-  if (kvt && need_vt) {
-    dmad::TransposeParams tt = tp;
-    tt.x = tv;
-    tt.y = ws + vt_bytes;
-    e = dmad::launch_transpose_pad(tt, BH, s);
+  if (need_vt) {
+    dmad::TransposeParams tp{};
+    tp.H = (int)H;
+    tp.D = (int)Dv;
+    tp.DP = (int)dvp;
+    tp.t[tp.count++] = {v, ws, v_strides[0], v_strides[1], v_strides[2], (int)Lk, (int)lkp};
+    if (kvt) tp.t[tp.count++] = {tv, ws + vt_bytes, v_strides[0], v_strides[1], v_strides[2], (int)Lk, (int)lkp};
+    e = dmad::launch_transpose_pad(tp, BH, s);
     if (e != hipSuccess) return fail(DMAD_ERR_HIP, "transpose launch: %s", hipGetErrorString(e));
   }
 
@@ -914,20 +914,23 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
   float* stats_bt = w.tgrad ? (float*)((char*)stats + w.stats) : nullptr;
 
   hipError_t e;
-  auto tr = [&](const void* x, const int64_t* st, char* y, int64_t L, int64_t LP) {
-    dmad::TransposeParams tp{x, y, st[0], st[1], st[2], (int)H, (int)L, (int)D, (int)LP, (int)dp};
-    return dmad::launch_transpose_pad(tp, (int)BH, s);
-  };
   // the full-derivative kernels of head dims other than 128, and the dO-only
   // ones of some head dims, read transposed copies of Q, dO (and Qd, dOd) and K
-  // (and Kd)
-  const bool need_tr = w.nq > 0;
-  if (need_tr && ((e = tr(q, q_strides, trq, Lq, lqp)) != hipSuccess || (e = tr(dout, do_strides, trdo, Lq, lqp)) != hipSuccess))
-    return fail(DMAD_ERR_HIP, "transpose launch: %s", hipGetErrorString(e));
-  if (w.nk > 0 && (e = tr(k, k_strides, trk, Lk, lkp)) != hipSuccess)
-    return fail(DMAD_ERR_HIP, "transpose launch: %s", hipGetErrorString(e));
-  if (need_tr && full && ((e = tr(tq, q_strides, trtq, Lq, lqp)) != hipSuccess || (e = tr(dto, do_strides, trdto, Lq, lqp)) != hipSuccess ||
-               (e = tr(tk, k_strides, trtk, Lk, lkp)) != hipSuccess))
+  // (and Kd), made in one launch
+  dmad::TransposeParams tp{};
+  tp.H = (int)H;
+  tp.D = (int)D;
+  tp.DP = (int)dp;
+  auto copy = [&](const void* x, const int64_t* st, char* y, int64_t L, int64_t LP) {
+    if (y != nullptr) tp.t[tp.count++] = {x, y, st[0], st[1], st[2], (int)L, (int)LP};
+  };
+  copy(q, q_strides, trq, Lq, lqp);
+  copy(dout, do_strides, trdo, Lq, lqp);
+  copy(k, k_strides, trk, Lk, lkp);
+  copy(tq, q_strides, trtq, Lq, lqp);
+  copy(dto, do_strides, trdto, Lq, lqp);
+  copy(tk, k_strides, trtk, Lk, lkp);
+  if ((e = dmad::launch_transpose_pad(tp, (int)BH, s)) != hipSuccess)
     return fail(DMAD_ERR_HIP, "transpose launch: %s", hipGetErrorString(e));
 
   const int ba = dmad::bwd_bmq((int)D, dmad::kBwdDoutOnly);
