@@ -352,10 +352,11 @@ def _check_device(*ts):
             )
 
 
-def jvp_attention_forward(q, k, v, tq, tk, tv, sm_scale, need_mu=True):
+def jvp_attention_forward(q, k, v, tq, tk, tv, sm_scale, need_mu=True, out=None):
     """Launch the forward(+JVP) kernel; returns (o, to, lse, mu).
 
-    ``tq is None`` selects the plain forward (to and mu are None).
+    ``tq is None`` selects the plain forward (to and mu are None). ``out``: where O goes, a
+    [B, H, Lq, Dv] tensor or view the kernels can write (default: a new contiguous one).
     """
     B, H, Lq, Dqk = q.shape
     Lk, Dv = v.shape[-2], v.shape[-1]
@@ -375,7 +376,7 @@ def jvp_attention_forward(q, k, v, tq, tk, tv, sm_scale, need_mu=True):
     k, tk = _pair(k, tk)
     v, tv = _pair(v, tv)
     dev = q.device
-    o = torch.empty((B, H, Lq, Dv), device=dev, dtype=q.dtype)
+    o = torch.empty((B, H, Lq, Dv), device=dev, dtype=q.dtype) if out is None else out
     to = torch.empty_like(o) if tq is not None else None
     lse = torch.empty((B, H, Lq), device=dev, dtype=torch.float32)
     mu = torch.empty_like(lse) if tq is not None else None
@@ -722,13 +723,32 @@ class _plain_attention(torch.autograd.Function):
         return _fwd_backward(ctx, dout, None)
 
 
-def plain_attention(q, k, v, sm_scale=None):
-    """softmax(sm_scale * q k^T) v for [B, H, L, D] tensors (gfx950 kernels), with backward."""
+def _plain_scale(q, k, v, sm_scale):
+    """The arguments' checks of plain attention; its softmax scale."""
     assert q.shape[:-2] == k.shape[:-2] and k.shape[:-2] == v.shape[:-2]
     assert k.shape[-2] == v.shape[-2] and q.shape[-1] == k.shape[-1]
     assert q.shape[-1] in _HEAD_DIMS and v.shape[-1] in _HEAD_DIMS
-    if sm_scale is None:
-        sm_scale = q.shape[-1] ** (-0.5)
+    return q.shape[-1] ** (-0.5) if sm_scale is None else sm_scale
+
+
+def plain_attention_bshd(q, k, v, sm_scale=None):
+    """plain_attention of [B, H, L, D] tensors as a contiguous [B, L, H, D] tensor. Where
+    nothing is kept for a backward the kernel writes that layout; otherwise O stays as the
+    backward reads it and the caller gets a copy (which it may then change in place)."""
+    keeps = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
+    if not keeps and _eager_call(q, k, v):
+        sm_scale = _plain_scale(q, k, v, sm_scale)
+        B, H, L, Dv = *q.shape[:-1], v.shape[-1]
+        if slice_fits(L, H * Dv, Dv, q.element_size()):
+            out = torch.empty((B, L, H, Dv), device=q.device, dtype=q.dtype)
+            jvp_attention_forward(q, k, v, None, None, None, sm_scale, out=out.transpose(1, 2))
+            return out
+    return plain_attention(q, k, v, sm_scale).transpose(1, 2).contiguous()
+
+
+def plain_attention(q, k, v, sm_scale=None):
+    """softmax(sm_scale * q k^T) v for [B, H, L, D] tensors (gfx950 kernels), with backward."""
+    sm_scale = _plain_scale(q, k, v, sm_scale)
     if _eager_call(q, k, v):
         if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
             return _plain_attention.apply(q, k, v, float(sm_scale))

@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import torch
 
-from .jvp_attention import plain_attention
+from .jvp_attention import plain_attention_bshd
 
 
 def attention(q, k, v, dropout_p=0.0, softmax_scale=None, q_scale=None, causal=False, deterministic=False):
@@ -37,5 +37,4 @@ def attention(q, k, v, dropout_p=0.0, softmax_scale=None, q_scale=None, causal=F
             f"dtype {q.dtype} is not supported by the gfx950 kernels (bfloat16, float16 or float32)")
     if q_scale is not None:
         q = q * q_scale
-    out = plain_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), softmax_scale)
-    return out.transpose(1, 2).contiguous()
+    return plain_attention_bshd(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), softmax_scale)

@@ -76,3 +76,21 @@ def test_second_derivatives_are_still_refused(gpu, plain):
     (gq,) = torch.autograd.grad(o.float().square().sum(), xs[:1], create_graph=True)
     with pytest.raises((RuntimeError, NotImplementedError)):
         torch.autograd.grad(gq.float().sum(), xs[:1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Lq,Lk,H", [(1, 3, 1), (130, 257, 3), (200, 4000, 2)])  # the last one splits
+def test_sdpa_writes_its_layout_without_a_copy(gpu, Lq, Lk, H, dtype):
+    """Without a backward the kernel writes BSHD; the values are those of the copied output."""
+    from dmad_amd.sdpa import attention
+
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn((2, L, H, 64), generator=g).to(dtype).to(gpu) for L in (Lq, Lk, Lk))
+    with torch.no_grad():
+        o = attention(q, k, v)
+    ref = attention(q.requires_grad_(True), k, v)
+    torch.cuda.synchronize()
+    assert o.is_contiguous() and o.shape == (2, Lq, H, 64) and torch.equal(o, ref)
+    if Lq > 1 and H > 1:  # else both layouts are one
+        ref.mul_(2.0).sum().backward()  # the tracked output is the caller's own to change
