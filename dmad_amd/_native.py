@@ -83,6 +83,11 @@ SIGNATURES = {
                                       _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
                                       _P, _P, _I64P, _P, _P, _F,
                                       _P, _P, _P, _I64, _I64, _P, _P, _I64, _I64, _P, _SZ, _P]),
+    "dmad_attn_magi_split_bytes": (_INT, [_INT, _I64, _I64, _I64, _I64, _I64, _I64, _SZP]),
+    "dmad_attn_jvp_fwd_magi_split": (_INT, [_INT, _INT, _I64, _I64, _I64, _I64, _I64, _I64,
+                                            _P, _P, _P, _P, _P, _P, _I64P, _I64P, _I64P,
+                                            _P, _P, _I64P, _P, _P, _F,
+                                            _P, _P, _P, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _SZ, _P, _SZ, _P]),
     "dmad_attn_fwd": (_INT, [_INT, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _P,
                              _I64P, _I64P, _I64P, _P, _I64P, _P, _F, _P, _SZ, _P]),
     "dmad_set_kernel_events": (_INT, [ctypes.POINTER(ctypes.c_void_p), _INT]),
@@ -199,6 +204,14 @@ def fwd_split_bytes(dtype: int, mode: int, B: int, H: int, Lq: int, Lk: int, Dqk
     their keys (0: it runs every tile whole)."""
     n = ctypes.c_size_t(0)
     check(lib().dmad_attn_fwd_split_bytes(dtype, mode, B, H, Lq, Lk, Dqk, Dv, ctypes.byref(n)))
+    return int(n.value)
+
+
+@functools.lru_cache(maxsize=1024)
+def magi_split_bytes(dtype: int, tasks: int, key_tiles: int, B: int, H: int, Dqk: int, Dv: int) -> int:
+    """The same for a block-sparse forward of ``tasks`` tasks of at most ``key_tiles`` key tiles."""
+    n = ctypes.c_size_t(0)
+    check(lib().dmad_attn_magi_split_bytes(dtype, tasks, key_tiles, B, H, Dqk, Dv, ctypes.byref(n)))
     return int(n.value)
 
 

@@ -109,6 +109,8 @@ __device__ __forceinline__ int magi_ntiles(const FwdParams& p, const MagiTask& t
   }
   return n;
 }
+// First tile of piece i of n of a task of `ntiles` tiles (split launches).
+__device__ __forceinline__ int magi_piece(int ntiles, int i, int n) { return (int)((int64_t)ntiles * i / n); }
 // Walks the key tiles of a task: current range r (clipped to [k0, k1)) and
 // the first key row of the current BN-key tile; past the last range it
 // points at row Lk and beyond (tiles of zeros, never used).
@@ -127,6 +129,19 @@ struct MagiCursor {
   __device__ __forceinline__ void next(const FwdParams& p, int bn) {
     start += bn;
     if (start >= k1 && r < r_end) {
+      ++r;
+      seek(p, bn);
+    }
+  }
+  // n tiles on
+  __device__ __forceinline__ void skip(const FwdParams& p, int bn, int n) {
+    while (n > 0 && r < r_end) {
+      const int left = (k1 + bn - 1) / bn - start / bn;  // tiles of this range
+      if (n < left) {
+        start += n * bn;
+        return;
+      }
+      n -= left;
       ++r;
       seek(p, bn);
     }

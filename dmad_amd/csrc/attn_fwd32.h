@@ -134,8 +134,8 @@ __device__ __forceinline__ void stage_store(const lds_char_t* region, int k, int
 // registers); two at D = 64, four for its dense plain forward (128 registers,
 // 32 KiB of LDS per workgroup; 1-2% faster than two, bitwise equal).
 //
-// SPLIT (64- and 128-wide heads, dense): the last work items of the grid run in
-// pieces of their key range (split.h); a piece sees its keys as the whole
+// SPLIT (64- and 128-wide heads): the last work items of the grid run in pieces of
+// their key range, or of their task's key tiles (split.h); a piece sees its keys as the whole
 // sequence and writes O~ / l, C~ / l, its logsumexp and mu as fp32 partials.
 template <typename T, int MODE, bool MAGI = false, int DH = 128, bool SPLIT = false>
 __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2) : 1) void attn_fwd32_kernel(
@@ -165,8 +165,30 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   int r_beg = 0, r_end = 0;   // key ranges of the group (MAGI)
   int lk = p.Lk, key0 = 0;    // keys of this workgroup (SPLIT: of its piece), the first one's row
   int part_slot = -1;         // SPLIT: partial block of this piece
-  static_assert(!SPLIT || (!MAGI && C::CHUNKS == 1 && DVC == D), "split launches: dense, all of V in one workgroup");
-  if constexpr (SPLIT) {
+  int skip = 0;               // MAGI, SPLIT: tiles of the task before this piece
+  static_assert(!SPLIT || (C::CHUNKS == 1 && DVC == D), "split launches: all of V in one workgroup");
+  if constexpr (SPLIT && MAGI) {
+    const SplitWork w = split_work(p.sp, 1, 0);
+    if (w.item < 0) return;
+    bh = w.item / p.T;
+    const MagiTask t = magi_task(p, w.item - bh * p.T, C::BM);
+    qt = t.row0 / C::BM;
+    q_lo = t.q_lo;
+    q_hi = t.q_hi;
+    r_beg = t.r_beg;
+    r_end = t.r_end;
+    ntiles = magi_ntiles(p, t, BN);
+    if (ntiles == 0) {
+      if (w.piece <= 0) magi_store_empty<T, D, C::JVP>(p, bh, t, C::BM);
+      return;
+    }
+    if (w.piece >= 0) {
+      part_slot = w.slot;
+      skip = magi_piece(ntiles, w.piece, p.sp.n);
+      ntiles = magi_piece(ntiles, w.piece + 1, p.sp.n) - skip;
+      if (ntiles == 0) return;  // the combining kernel leaves it out
+    }
+  } else if constexpr (SPLIT) {
     const int nqt = (p.Lq + C::BM - 1) / C::BM;
     const SplitWork w = split_work(p.sp, p.xcd_order, (p.Lk + BN - 1) / BN);
     if (w.item < 0) return;
@@ -241,7 +263,7 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   // V (Vd) resources start at this workgroup's column chunk
   const uint32_t v_bytes = (uint32_t)(((int64_t)(lk - 1) * p.v_sl + DVC) * 2);
   int64_t khead = b * p.k_sb + h * p.k_sh, vhead = b * p.v_sb + h * p.v_sh + chunk * DVC;
-  if constexpr (SPLIT) {
+  if constexpr (SPLIT && !MAGI) {
     khead += (int64_t)key0 * p.k_sl;
     vhead += (int64_t)key0 * p.v_sl;
   }
@@ -512,6 +534,7 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   };
   MagiCursor ci{r_beg, r_end, 0, 0, 0};  // MAGI: tile requested next
   if constexpr (MAGI) ci.seek(p, BN);
+  if constexpr (MAGI && SPLIT) ci.skip(p, BN, skip);
   MagiCursor cm = ci;  // MAGI: tile whose softmax runs next
 
   // step i (i + 1 < ntiles, i % 4 == kk): phase A on tile i+1's K, softmax of

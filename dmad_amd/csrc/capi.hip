@@ -308,6 +308,24 @@ dmad::SplitPlan plan_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_
   return dmad::plan_split(items, steps, fwd_split_cost(mode, Dqk));
 }
 
+// The split of a block-sparse forward's last tasks, whose lengths the host does not
+// see: `key_tiles`, the most 32-key tiles one of them walks, says what a split saves
+// (0: unknown, none). Each split task is cut in equal shares of its own tiles. As
+// the dense forward, both modes split alike.
+dmad::SplitPlan plan_magi_split(int dtype, int64_t tasks, int64_t key_tiles, int64_t B, int64_t H, int64_t Dqk,
+                                int64_t Dv) {
+  dmad::SplitPlan none;
+  none.whole = none.grid = tasks * B * H;
+  if (dtype == DMAD_F32 || key_tiles <= 0 || !dmad::fwd32_supported((int)Dqk, (int)Dv)) return none;
+  return dmad::plan_split(tasks * B * H, key_tiles, fwd_split_cost(DMAD_FWD_JVP, Dqk), true);
+}
+
+dmad::FwdLaunchFn pick_fwd_magi_split(int dtype, int64_t d, int mode) {
+  if (dtype == DMAD_BF16) return dmad::fwd32_magi_split_select<__bf16>(mode, (int)d);
+  if (dtype == DMAD_F16) return dmad::fwd32_magi_split_select<_Float16>(mode, (int)d);
+  return nullptr;
+}
+
 dmad::FwdLaunchFn pick_fwd_split(int dtype, int64_t d, int mode) {
   if (dtype == DMAD_F32) {
     switch (d) {
@@ -327,6 +345,7 @@ dmad::FwdLaunchFn pick_fwd_split(int dtype, int64_t d, int mode) {
 struct MagiArgs {
   const int32_t *q_ranges, *k_ranges, *qk_map, *task_group, *task_qtile;
   int64_t G, R, T;
+  int64_t key_tiles;  // most 32-key tiles of a task, 0 if not known
 };
 
 dmad::BwdLaunchFn pick_bwd(int dtype, int64_t d, int mode) {
@@ -655,10 +674,12 @@ int fwd_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, 
 
   // with room for the partials, the last query tiles run in pieces of their keys
   dmad::SplitPlan sp;
-  if (split_ws != nullptr && mg == nullptr) {
-    sp = plan_fwd_split(dtype, mode, B, H, Lq, Lk, Dqk, Dv);
+  if (split_ws != nullptr) {
+    sp = mg ? plan_magi_split(dtype, mg->T, mg->key_tiles, B, H, Dqk, Dv)
+            : plan_fwd_split(dtype, mode, B, H, Lq, Lk, Dqk, Dv);
     if (sp.rest == 0 || (int64_t)split_bytes < sp.bytes) sp = dmad::SplitPlan{};
-    else if ((fn = pick_fwd_split(dtype, Dqk, mode)) == nullptr) return fail(DMAD_ERR_UNSUPPORTED, "no split kernel");
+    else if ((fn = mg ? pick_fwd_magi_split(dtype, Dqk, mode) : pick_fwd_split(dtype, Dqk, mode)) == nullptr)
+      return fail(DMAD_ERR_UNSUPPORTED, "no split kernel");
   }
 
   hipStream_t s = (hipStream_t)stream;
@@ -1165,13 +1186,14 @@ int dmad_attn_jvp_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_t L
                   o_strides, lse, mu, sm_scale, workspace, workspace_bytes, split_ws, split_bytes, stream, nullptr);
 }
 
-int dmad_attn_jvp_fwd_magi(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv,
-                           const void* q, const void* k, const void* v, const void* tq, const void* tk, const void* tv,
-                           const int64_t q_strides[4], const int64_t k_strides[4], const int64_t v_strides[4],
-                           void* o, void* to, const int64_t o_strides[4], float* lse, float* mu, float sm_scale,
-                           const int32_t* q_ranges, const int32_t* k_ranges, const int32_t* qk_map, int64_t G,
-                           int64_t R, const int32_t* task_group, const int32_t* task_qtile, int64_t T,
-                           int64_t block_m, void* workspace, size_t workspace_bytes, void* stream) {
+static int fwd_magi_impl(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv,
+                         const void* q, const void* k, const void* v, const void* tq, const void* tk, const void* tv,
+                         const int64_t q_strides[4], const int64_t k_strides[4], const int64_t v_strides[4], void* o,
+                         void* to, const int64_t o_strides[4], float* lse, float* mu, float sm_scale,
+                         const int32_t* q_ranges, const int32_t* k_ranges, const int32_t* qk_map, int64_t G, int64_t R,
+                         const int32_t* task_group, const int32_t* task_qtile, int64_t T, int64_t block_m,
+                         int64_t key_tiles, void* workspace, size_t workspace_bytes, void* split_ws,
+                         size_t split_bytes, void* stream) {
   if (block_m != dmad::kMagiBlockM)
     return fail(DMAD_ERR_UNSUPPORTED, "tasks must be built for %d-query tiles, got BLOCK_M=%lld", dmad::kMagiBlockM,
                 (long long)block_m);
@@ -1180,9 +1202,44 @@ int dmad_attn_jvp_fwd_magi(int dtype, int mode, int64_t B, int64_t H, int64_t Lq
   if (q_ranges == nullptr || qk_map == nullptr || (R > 0 && k_ranges == nullptr) ||
       (T > 0 && (task_group == nullptr || task_qtile == nullptr)))
     return fail(DMAD_ERR_INVALID, "block-sparse tables: null pointer");
-  const MagiArgs mg{q_ranges, k_ranges, qk_map, task_group, task_qtile, G, R, T};
+  const MagiArgs mg{q_ranges, k_ranges, qk_map, task_group, task_qtile, G, R, T, key_tiles};
   return fwd_impl(dtype, mode, B, H, Lq, Lk, Dqk, Dv, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to,
-                  o_strides, lse, mu, sm_scale, workspace, workspace_bytes, nullptr, 0, stream, &mg);
+                  o_strides, lse, mu, sm_scale, workspace, workspace_bytes, split_ws, split_bytes, stream, &mg);
+}
+
+int dmad_attn_jvp_fwd_magi(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv,
+                           const void* q, const void* k, const void* v, const void* tq, const void* tk, const void* tv,
+                           const int64_t q_strides[4], const int64_t k_strides[4], const int64_t v_strides[4],
+                           void* o, void* to, const int64_t o_strides[4], float* lse, float* mu, float sm_scale,
+                           const int32_t* q_ranges, const int32_t* k_ranges, const int32_t* qk_map, int64_t G,
+                           int64_t R, const int32_t* task_group, const int32_t* task_qtile, int64_t T,
+                           int64_t block_m, void* workspace, size_t workspace_bytes, void* stream) {
+  return fwd_magi_impl(dtype, mode, B, H, Lq, Lk, Dqk, Dv, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to,
+                       o_strides, lse, mu, sm_scale, q_ranges, k_ranges, qk_map, G, R, task_group, task_qtile, T,
+                       block_m, 0, workspace, workspace_bytes, nullptr, 0, stream);
+}
+
+int dmad_attn_magi_split_bytes(int dtype, int64_t tasks, int64_t key_tiles, int64_t B, int64_t H, int64_t Dqk,
+                               int64_t Dv, size_t* bytes) {
+  if (bytes == nullptr) return fail(DMAD_ERR_INVALID, "bytes: null pointer");
+  if (tasks < 0 || key_tiles < 0 || B < 0 || H < 0 || !head_dim_ok(Dqk) || !head_dim_ok(Dv)) return fail(DMAD_ERR_INVALID, "bad sizes");
+  *bytes = (size_t)plan_magi_split(dtype, tasks, key_tiles, B, H, Dqk, Dv).bytes;
+  return ok();
+}
+
+int dmad_attn_jvp_fwd_magi_split(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk,
+                                 int64_t Dv, const void* q, const void* k, const void* v, const void* tq,
+                                 const void* tk, const void* tv, const int64_t q_strides[4],
+                                 const int64_t k_strides[4], const int64_t v_strides[4], void* o, void* to,
+                                 const int64_t o_strides[4], float* lse, float* mu, float sm_scale,
+                                 const int32_t* q_ranges, const int32_t* k_ranges, const int32_t* qk_map, int64_t G,
+                                 int64_t R, const int32_t* task_group, const int32_t* task_qtile, int64_t T,
+                                 int64_t block_m, int64_t key_tiles, void* workspace, size_t workspace_bytes,
+                                 void* split_ws, size_t split_bytes, void* stream) {
+  return fwd_magi_impl(dtype, mode, B, H, Lq, Lk, Dqk, Dv, q, k, v, tq, tk, tv, q_strides, k_strides, v_strides, o, to,
+                       o_strides, lse, mu, sm_scale, q_ranges, k_ranges, qk_map, G, R, task_group, task_qtile, T,
+                       block_m, key_tiles < 0 ? 0 : key_tiles, workspace, workspace_bytes, split_ws, split_bytes,
+                       stream);
 }
 
 int dmad_attn_fwd(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv, const void* q,

@@ -34,8 +34,7 @@ static hipError_t f32_fwd_split_launch(const FwdParams& p, int grid, hipStream_t
                      dim3(F32FwdCfg<D, D, MODE, false>::NT), 0, s, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  FwdCombineParams c{p.sp, p.o, p.to, p.lse, p.mu, p.o_sb, p.o_sh, p.o_sl, p.H, p.Lq};
-  hipLaunchKernelGGL((fwd_combine_kernel<float, D, MODE != kFwdPlain, 16>), dim3(8 * p.sp.rest), dim3(256), 0, s, c);
+  hipLaunchKernelGGL((fwd_combine_kernel<float, D, MODE != kFwdPlain, 16>), dim3(8 * p.sp.rest), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 

@@ -28,14 +28,22 @@ static hipError_t fwd32_split_launch(const FwdParams& p, int grid, hipStream_t s
   hipLaunchKernelGGL((attn_fwd32_kernel<T, MODE, false, D, true>), dim3(grid), dim3(256), 0, s, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  FwdCombineParams c{p.sp, p.o, p.to, p.lse, p.mu, p.o_sb, p.o_sh, p.o_sl, p.H, p.Lq};
-  hipLaunchKernelGGL((fwd_combine_kernel<T, D, MODE != kFwdPlain>), dim3(4 * p.sp.rest), dim3(256), 0, s, c);
+  hipLaunchKernelGGL((fwd_combine_kernel<T, D, MODE != kFwdPlain>), dim3(4 * p.sp.rest), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
 template <typename T, int MODE, int D>
 static hipError_t fwd32_magi_launch(const FwdParams& p, int grid, hipStream_t s) {
   hipLaunchKernelGGL((attn_fwd32_kernel<T, MODE, true, D>), dim3(grid), dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+
+template <typename T, int MODE, int D>
+static hipError_t fwd32_magi_split_launch(const FwdParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_fwd32_kernel<T, MODE, true, D, true>), dim3(grid), dim3(256), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((fwd_combine_kernel<T, D, true, 32, true>), dim3(4 * p.sp.rest), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
@@ -77,6 +85,20 @@ static FwdLaunchFn fwd32_split_mode(int mode) {
 template <>
 FwdLaunchFn fwd32_split_select<Elt>(int mode, int d) {
   return d == 64 ? fwd32_split_mode<64>(mode) : d == 128 ? fwd32_split_mode<128>(mode) : nullptr;
+}
+
+template <int D>
+static FwdLaunchFn fwd32_magi_split_mode(int mode) {
+  switch (mode) {
+    case kFwdJvp: return &fwd32_magi_split_launch<Elt, kFwdJvp, D>;
+    case kFwdJvpQOnly: return &fwd32_magi_split_launch<Elt, kFwdJvpQOnly, D>;
+    default: return nullptr;
+  }
+}
+
+template <>
+FwdLaunchFn fwd32_magi_split_select<Elt>(int mode, int d) {
+  return d == 64 ? fwd32_magi_split_mode<64>(mode) : d == 128 ? fwd32_magi_split_mode<128>(mode) : nullptr;
 }
 
 template <>

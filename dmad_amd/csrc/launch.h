@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include "attn_fwd.h"
 #include "attn_fwd32.h"
+#include "fwd_combine.h"
 #include "attn_fwd32_x2.h"
 #include "attn_bwd.h"
 #include "attn_bwd_dq.h"
@@ -32,6 +33,11 @@ template <typename T>
 FwdLaunchFn fwd32_split_select(int mode, int d);
 template <> FwdLaunchFn fwd32_split_select<__bf16>(int, int);
 template <> FwdLaunchFn fwd32_split_select<_Float16>(int, int);
+// The same for the block-sparse forward: the last tasks in pieces of their tiles.
+template <typename T>
+FwdLaunchFn fwd32_magi_split_select(int mode, int d);
+template <> FwdLaunchFn fwd32_magi_split_select<__bf16>(int, int);
+template <> FwdLaunchFn fwd32_magi_split_select<_Float16>(int, int);
 
 // Two-workgroups-per-CU forward (attn_fwd32_x2_kernel; mode kFwdJvpQOnly,
 // 128-wide heads): one workgroup per 128-query tile.

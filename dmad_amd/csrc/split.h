@@ -114,12 +114,12 @@ inline double split_makespan(const SplitCost& k, int64_t a, double la, int64_t b
 
 // How to run `items` work items of `steps` steps: in full rounds, then the rest in
 // the pieces that finish soonest by the costs above, where that saves at least a
-// twentieth of the launch and 8 us: the second kernel and its scratch cost the host
+// twentieth of the launch and 8 us (even_only: in pieces of one length): the second kernel and its scratch cost the host
 // 4-5 us, and calls that short wait for the host (a training call of two 64-wide
 // heads of 999 tokens: 45 us of kernels split, 67 whole, in 200 us of host time,
 // 12 of them for the three splits). The partials are written and read once, at about
 // 3.3 TB/s, by a second kernel that takes 5 us at least (all measured).
-inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k) {
+inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k, bool even_only = false) {
   SplitPlan pl;
   pl.whole = items;
   pl.grid = items;
@@ -135,7 +135,7 @@ inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k) {
     // the shorter last piece runs in the slots the n - 1 long ones leave free
     const int64_t left = slots - (n - 1) * rest;
     int64_t lens[2] = {even, 0};
-    if (left > 0 && left < rest) {
+    if (!even_only && left > 0 && left < rest) {
       const int64_t q = (rest + left - 1) / left;
       lens[1] = (steps * q + (n - 1) * q) / ((n - 1) * q + 1);
     }
@@ -173,112 +173,6 @@ struct FwdPart {
   static constexpr int STATS = WAVES * NT * TILE;
   static constexpr int FLOATS = STATS + WAVES * 2 * ROWS;
 };
-
-struct FwdCombineParams {
-  SplitParams sp;
-  void* o;
-  void* to;
-  float* lse;
-  float* mu;
-  int64_t o_sb, o_sh, o_sl;
-  int H, Lq;
-};
-
-// One workgroup per wave tile (ROWS queries) of a split item; thread = (lane of the
-// tile, one of 4 groups of columns). Bound by reading the partials once.
-template <typename T, int D, bool JVP, int ROWS = 32>
-__global__ __launch_bounds__(256) void fwd_combine_kernel(FwdCombineParams p) {
-  using P = FwdPart<D, JVP, ROWS>;
-  constexpr int GROUPS = ROWS * D / 256;          // 16-byte column groups of a tile's lane
-  constexpr int NG = (GROUPS + 3) / 4;            // ... per thread: groups grp, grp + 4, ...
-  constexpr int U = NG * (JVP ? 2 : 1) > 8 ? 2 : 4;  // pieces in flight
-  const int item = (int)blockIdx.x / P::WAVES, wave = (int)blockIdx.x % P::WAVES;
-  const int lane = lane_id(), col = lane % ROWS, half = lane / ROWS, grp = threadIdx.x >> 6;
-  if (grp >= GROUPS) return;
-  const int nqt = (p.Lq + 127) / 128;
-  const int work = p.sp.whole + item, bh = work / nqt, qt = work - bh * nqt;
-  const int query = qt * 128 + wave * ROWS + col;
-  const float* part = p.sp.part + (int64_t)item * p.sp.n * P::FLOATS;
-  const float* st = part + P::STATS + wave * 2 * ROWS + col;
-  // pieces are taken U at a time with all of their loads in flight together (the
-  // partials come from other XCDs' workgroups, about a microsecond away); past
-  // the last piece the last one is read again and left out
-  const int n = p.sp.n;
-  float m = -__builtin_inff();
-  for (int i = 0; i < n; i += 8) {
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = st[(int64_t)min(i + u, n - 1) * P::FLOATS];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) m = fmaxf(m, v[u]);
-  }
-  float w = 0.f, mu = 0.f;
-  f32x4_t o[NG], c[NG];
-#pragma unroll
-  for (int g = 0; g < NG; ++g) o[g] = c[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < n; i += U) {
-    f32x4_t ov[U][NG], cv[U][NG];
-    float lse2[U], mus[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float* pi = part + (int64_t)min(i + u, n - 1) * P::FLOATS;
-      lse2[u] = pi[P::STATS + wave * 2 * ROWS + col];
-      if constexpr (JVP) mus[u] = pi[P::STATS + wave * 2 * ROWS + ROWS + col];
-      const float* tile = pi + wave * P::NT * P::TILE;
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        const int j = 4 * g + grp < GROUPS ? 4 * g + grp : grp;
-        ov[u][g] = split_get(tile, lane, j);
-        if constexpr (JVP) cv[u][g] = split_get(tile + P::TILE, lane, j);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (i + u >= n) break;
-      const float wi = fast_exp2(lse2[u] - m);
-      w += wi;
-      if constexpr (JVP) mu += wi * mus[u];
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          o[g][e] = fmaf(wi, ov[u][g][e], o[g][e]);
-          if constexpr (JVP) c[g][e] = fmaf(wi, cv[u][g][e], c[g][e]);
-        }
-      }
-    }
-  }
-  if (query >= p.Lq) return;
-  const float inv = 1.0f / w;
-  mu *= inv;
-  const int b = bh / p.H, h = bh - b * p.H;
-  const int64_t off = b * p.o_sb + h * p.o_sh + (int64_t)query * p.o_sl;
-#pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    if (4 * g + grp >= GROUPS) break;
-    const int dc = (4 * g + grp) * (256 / ROWS) + 4 * half;  // a group is 256 / ROWS columns wide
-    f32x4_t ov, tv;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      ov[e] = o[g][e] * inv;
-      tv[e] = c[g][e] * inv - mu * ov[e];
-    }
-    if constexpr (std::is_same<T, float>::value) {
-      *(f32x4_t*)((float*)p.o + off + dc) = ov;
-      if constexpr (JVP) *(f32x4_t*)((float*)p.to + off + dc) = tv;
-    } else {
-      *(u32x2_t*)((char*)p.o + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(ov[0], ov[1]), Elem<T>::pack2(ov[2], ov[3])};
-      if constexpr (JVP)
-        *(u32x2_t*)((char*)p.to + (off + dc) * 2) = u32x2_t{Elem<T>::pack2(tv[0], tv[1]), Elem<T>::pack2(tv[2], tv[3])};
-    }
-  }
-  if (half == 0 && grp == 0) {
-    const int64_t si = (int64_t)bh * p.Lq + query;
-    p.lse[si] = (m + __builtin_log2f(w)) * 0.6931471805599453f;
-    if constexpr (JVP) p.mu[si] = mu;
-  }
-}
 
 // ---------------------------------------------------------------- backward
 // Partial block of a backward pass: [waves][tensors][32 x D] accumulator tiles,

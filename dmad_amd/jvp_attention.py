@@ -434,15 +434,17 @@ def jvp_attention_forward_magi(q, k, v, tq, tk, tv, sm_scale, magi_mask):
     mu = torch.empty_like(lse)
     lib = nat.lib()
     ws_ptr, ws_size, ws = nat.workspace(_fwd_ws_bytes(q.dtype, mode, B, H, Lk, Dqk, Dv), dev)
+    key_tiles = int(getattr(magi_mask, "key_tiles", 0))
+    sp_ptr, sp_size, sp = _split_workspace(nat.magi_split_bytes(code, T, key_tiles, B, H, Dqk, Dv), dev)
     nat.check(
-        lib.dmad_attn_jvp_fwd_magi(
+        lib.dmad_attn_jvp_fwd_magi_split(
             code, mode, B, H, Lq, Lk, Dqk, Dv,
             nat.ptr(q), nat.ptr(k), nat.ptr(v), nat.ptr(tq), nat.ptr(tk), nat.ptr(tv),
             nat.strides4(q), nat.strides4(k), nat.strides4(v),
             nat.ptr(o), nat.ptr(to), nat.strides4(o), nat.ptr(lse), nat.ptr(mu), float(sm_scale),
             nat.ptr(q_unique), nat.ptr(k_flat), nat.ptr(qk_map), G, R,
-            nat.ptr(task_group), nat.ptr(task_qtile), T, mm.KERNEL_BLOCK_M,
-            ws_ptr, ws_size, nat.stream_ptr(dev),
+            nat.ptr(task_group), nat.ptr(task_qtile), T, mm.KERNEL_BLOCK_M, key_tiles,
+            ws_ptr, ws_size, sp_ptr, sp_size, nat.stream_ptr(dev),
         )
     )
     return o, to, lse, mu

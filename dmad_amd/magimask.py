@@ -253,6 +253,9 @@ class MagiMask:
     G: int
     T: int
     BLOCK_M: int
+    # most 32-key tiles a query group walks (0: not known): what the launch goes by when it
+    # decides whether to cut the last tasks; results do not depend on it
+    key_tiles: int = 0
 
 
 def prepare_magi_csr_and_tasks(q_ranges: torch.Tensor, k_ranges: torch.Tensor, Q_real: int, KV_real: int,
@@ -268,9 +271,12 @@ def prepare_magi_csr_and_tasks(q_ranges: torch.Tensor, k_ranges: torch.Tensor, Q
         assert qu[i, 1] == qu[i + 1, 0], \
             f"query groups {i} and {i + 1} do not meet: {qu[i].tolist()} then {qu[i + 1].tolist()}"
     task_group, task_qtile = build_qtile_tasks(q_unique, Q_real=Q_real, BLOCK_M=BLOCK_M)
+    kf = _host(k_flat)
+    tiles = np.append((kf[:, 1] + 31) // 32 - kf[:, 0] // 32, 0)
+    most = int(np.add.reduceat(tiles, qk_map.detach().cpu().numpy()[:-1]).max())
     return MagiMask(q_unique=q_unique.contiguous(), k_flat=k_flat.contiguous(), qk_map=qk_map.contiguous(),
                     task_group=task_group, task_qtile=task_qtile, G=int(qu.shape[0]), T=int(task_group.numel()),
-                    BLOCK_M=int(BLOCK_M))
+                    BLOCK_M=int(BLOCK_M), key_tiles=most)
 
 
 def csr_to_dense(q_unique, k_flat, qk_map, Q: int, KV: int) -> torch.Tensor:

@@ -130,6 +130,25 @@ int dmad_attn_jvp_fwd_magi(int dtype, int mode, int64_t B, int64_t H, int64_t Lq
                            int64_t block_m, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * dmad_attn_jvp_fwd_magi with scratch for partials, as dmad_attn_jvp_fwd_split:
+ * the tasks that do not fill a round over the chip are cut into equal shares of
+ * the key tiles each walks. key_tiles is the most 32-key tiles a task walks (it
+ * decides whether and how far to cut, not what is computed; 0: not known, no
+ * task is cut).
+ */
+int dmad_attn_magi_split_bytes(int dtype, int64_t tasks, int64_t key_tiles, int64_t B, int64_t H, int64_t Dqk,
+                               int64_t Dv, size_t* bytes);
+int dmad_attn_jvp_fwd_magi_split(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk,
+                                 int64_t Dv, const void* q, const void* k, const void* v, const void* tq,
+                                 const void* tk, const void* tv, const int64_t q_strides[4],
+                                 const int64_t k_strides[4], const int64_t v_strides[4], void* o, void* to,
+                                 const int64_t o_strides[4], float* lse, float* mu, float sm_scale,
+                                 const int32_t* q_ranges, const int32_t* k_ranges, const int32_t* qk_map, int64_t G,
+                                 int64_t R, const int32_t* task_group, const int32_t* task_qtile, int64_t T,
+                                 int64_t block_m, int64_t key_tiles, void* workspace, size_t workspace_bytes,
+                                 void* split_ws, size_t split_bytes, void* stream);
+
+/*
  * Plain forward (O and LSE), the attention used by the non-JVP Wan forward
  * (train/wan/rcm/utils/jvp_helper.py:305-308 and rcm/utils/attention.py:120-167).
  */

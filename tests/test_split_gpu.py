@@ -152,3 +152,48 @@ def test_split_backward(gpu, monkeypatch, B, H, Lq, Lk, D, full, dtype):
     ref = orc.grads_full(*xs) if full else orc.grads_dout_only(*xs[:3], xs[6])
     for name, a, w, r in zip(names, got, whole, ref):
         _no_worse(name, a, w, r)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kv_tangents", [True, False])
+@pytest.mark.parametrize("hint", [60, 3000])  # a few pieces per task; more pieces than some tasks have tiles
+def test_split_block_sparse_forward(gpu, hint, kv_tangents, D, dtype):
+    """Tasks of unequal lengths, ranges off the tile grid, a group without keys and rows that no
+    task covers: split (the mask's length hint set by hand) against whole and the oracle."""
+    import dataclasses
+
+    from dmad_amd import _native as nat
+    from dmad_amd import magimask as mm
+    from dmad_amd.jvp_attention import jvp_attention_forward_magi
+    from oracle import magi as om
+
+    print(f"case split magi hint={hint} kv={kv_tangents} D={D} {dtype}", flush=True)
+    B, H, Lq, Lk = 1, 2, 700, 1300
+    groups = [(0, 200, [(0, 40)]), (200, 330, [(33, 500), (777, 1300)]), (330, 400, []), (400, 650, [(5, 1290)])]
+    keys = [r for g in groups for r in g[2]]
+    first = [sum(len(g[2]) for g in groups[:i]) for i in range(len(groups) + 1)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)  # noqa: E731
+    qu = i32([[g[0], g[1]] for g in groups])
+    tg, tq_ = mm.build_qtile_tasks(qu, Lq, 128)
+    mask = mm.MagiMask(qu, i32(keys), i32(first), tg, tq_, len(groups), int(tg.numel()), 128)
+    code = nat.dtype_code(dtype)
+    split = dataclasses.replace(mask, key_tiles=hint)
+    assert nat.magi_split_bytes(code, mask.T, hint, B, H, D, D) > 0
+    q, k, v, tq, tk, tv = _draw(gpu, D, B, H, Lq, Lk, D, dtype)
+    tk, tv = (tk, tv) if kv_tangents else (None, None)
+    whole = jvp_attention_forward_magi(q, k, v, tq, tk, tv, D ** -0.5, mask)
+    got = jvp_attention_forward_magi(q, k, v, tq, tk, tv, D ** -0.5, split)
+    again = jvp_attention_forward_magi(q, k, v, tq, tk, tv, D ** -0.5, split)
+    torch.cuda.synchronize()
+    allow = torch.zeros(Lq, Lk, dtype=torch.bool)
+    for a, b, rs in groups:
+        for s, e in rs:
+            allow[a:b, s:e] = True
+    xs = [t.cpu() for t in (q, k, v, tq)] + [(t if t is not None else torch.zeros_like(k)).cpu() for t in (tk, tv)]
+    ref = om.masked_jvp(*xs, allow, D ** -0.5)
+    for name, a, b, w, r in zip(("o", "to", "lse", "mu"), got, again, whole, ref):
+        assert torch.equal(a[:, :, :650], b[:, :, :650]), name  # rows from 650 on are nobody's
+        keep = torch.cat([torch.arange(330), torch.arange(400, 650)])
+        _no_worse(name, a[:, :, keep], w[:, :, keep], r[:, :, keep])
+        assert torch.equal(a[:, :, 330:400], w[:, :, 330:400]), name  # no keys: zeros, LSE -inf
