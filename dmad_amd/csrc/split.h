@@ -85,6 +85,7 @@ struct SplitPlan {
 
 constexpr int kSplitCus = 256;
 constexpr int kSplitMaxPieces = 64;
+constexpr int64_t kSplitMaxBytes = (int64_t)128 << 20;  // partials of one launch
 
 // Time of `a` workgroups of la steps followed by `b` of lb <= la, dealt to the
 // free slots in that order.
@@ -129,7 +130,7 @@ inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k, bo
   const double as_is = split_makespan(k, rest, (double)steps, 0, 0.);
   const double least = 0.05 * (as_is + (double)rounds * round);
   double best = as_is - (least > 8. ? least : 8.);
-  for (int64_t n = 2; n <= kSplitMaxPieces && n <= steps; ++n) {
+  for (int64_t n = 2; n <= kSplitMaxPieces && n <= steps && rest * n * k.part_bytes <= kSplitMaxBytes; ++n) {
     const double extra = 5. + 2. * (double)(rest * n) * k.part_bytes / 3.3e6;
     const int64_t even = (steps + n - 1) / n;
     // the shorter last piece runs in the slots the n - 1 long ones leave free

@@ -171,7 +171,7 @@ def _backward_workspace(code: int, ws_mode: int, B: int, H: int, Lq: int, Lk: in
 
 def _split_workspace(nbytes: int, device):
     """(pointer, size, owner) of the partials of a split launch. The split only saves time:
-    without room for its partials (at most 64 MiB or so) every tile runs whole."""
+    without room for its partials (at most 128 MiB) every tile runs whole."""
     if nbytes == 0:
         return None, 0, None
     try:

@@ -179,6 +179,13 @@ def merge_k_ranges(q_ranges: torch.Tensor, k_ranges: torch.Tensor, KV_real: int)
     """Rows sorted by query range; per query range the key ranges clipped to
     [0, KV_real], empty ones dropped, sorted by start and merged where they
     overlap or touch (train/wan/rcm/utils/magimask.py:127-184)."""
+    arr, dev = _merged(q_ranges, k_ranges, KV_real), q_ranges.device
+    return (torch.tensor(arr[:, :2], device=dev, dtype=torch.int32),
+            torch.tensor(arr[:, 2:], device=dev, dtype=torch.int32))
+
+
+def _merged(q_ranges: torch.Tensor, k_ranges: torch.Tensor, KV_real: int) -> np.ndarray:
+    """merge_k_ranges on the host: rows (q0, q1, k0, k1)."""
     assert q_ranges.shape == k_ranges.shape and q_ranges.ndim == 2 and q_ranges.shape[1] == 2
     qs, ks = _host(q_ranges), _host(k_ranges)
     order = np.lexsort((qs[:, 1], qs[:, 0]))  # stable: by q0, then q1
@@ -203,10 +210,7 @@ def merge_k_ranges(q_ranges: torch.Tensor, k_ranges: torch.Tensor, KV_real: int)
                 lo, hi = a, b
         out.append((q0, q1, lo, hi))
         i = j
-    arr = np.asarray(out, dtype=np.int64).reshape(-1, 4)
-    dev = q_ranges.device
-    return (torch.tensor(arr[:, :2], device=dev, dtype=torch.int32),
-            torch.tensor(arr[:, 2:], device=dev, dtype=torch.int32))
+    return np.asarray(out, dtype=np.int64).reshape(-1, 4)
 
 
 def group_q_ranges_csr(q_ranges: torch.Tensor, k_ranges: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -262,21 +266,23 @@ def prepare_magi_csr_and_tasks(q_ranges: torch.Tensor, k_ranges: torch.Tensor, Q
                                BLOCK_M: int = KERNEL_BLOCK_M) -> MagiMask:
     """Merge, group, check that the query groups partition [0, Q_real), build tasks
     (train/wan/rcm/utils/magimask.py:265-283). BLOCK_M defaults to the kernels' 128."""
-    q_ranges, k_ranges = merge_k_ranges(q_ranges, k_ranges, KV_real=KV_real)
-    q_unique, k_flat, qk_map = group_q_ranges_csr(q_ranges, k_ranges)
-    qu = _host(q_unique)
+    rows, dev = _merged(q_ranges, k_ranges, KV_real), q_ranges.device
+    new = np.flatnonzero(np.append(True, (rows[1:, :2] != rows[:-1, :2]).any(axis=1))) if len(rows) else np.zeros(0, int)
+    qu = rows[new, :2]
     assert len(qu) > 0 and qu[0, 0] == 0 and qu[-1, 1] == Q_real, \
         f"the query groups must start at row 0 and end at row {Q_real} (Q_real)"
     for i in range(len(qu) - 1):
         assert qu[i, 1] == qu[i + 1, 0], \
             f"query groups {i} and {i + 1} do not meet: {qu[i].tolist()} then {qu[i + 1].tolist()}"
-    task_group, task_qtile = build_qtile_tasks(q_unique, Q_real=Q_real, BLOCK_M=BLOCK_M)
-    kf = _host(k_flat)
-    tiles = np.append((kf[:, 1] + 31) // 32 - kf[:, 0] // 32, 0)
-    most = int(np.add.reduceat(tiles, qk_map.detach().cpu().numpy()[:-1]).max())
-    return MagiMask(q_unique=q_unique.contiguous(), k_flat=k_flat.contiguous(), qk_map=qk_map.contiguous(),
-                    task_group=task_group, task_qtile=task_qtile, G=int(qu.shape[0]), T=int(task_group.numel()),
-                    BLOCK_M=int(BLOCK_M), key_tiles=most)
+    task_group, task_qtile = _tasks(qu, Q_real, BLOCK_M)
+    most = np.add.reduceat((rows[:, 3] + 31) // 32 - rows[:, 2] // 32, new).max()
+
+    def table(x):
+        return torch.tensor(x, device=dev, dtype=torch.int32)
+
+    return MagiMask(q_unique=table(qu), k_flat=table(rows[:, 2:]), qk_map=table(np.append(new, len(rows))),
+                    task_group=table(task_group), task_qtile=table(task_qtile), G=len(qu), T=len(task_group),
+                    BLOCK_M=int(BLOCK_M), key_tiles=int(most))
 
 
 def csr_to_dense(q_unique, k_flat, qk_map, Q: int, KV: int) -> torch.Tensor:

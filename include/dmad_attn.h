@@ -82,7 +82,7 @@ int dmad_attn_jvp_fwd(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int
 /*
  * Bytes of partials with which dmad_attn_jvp_fwd_split runs the last query
  * tiles of these sizes in pieces of their keys (0: it would not; at most
- * about 70 MB).
+ * 128 MiB).
  */
 int dmad_attn_fwd_split_bytes(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk,
                               int64_t Dv, size_t* bytes);
