@@ -55,6 +55,14 @@ def test_full_rounds_and_other_head_dims_stay_whole():
     assert nat.magi_split_bytes(BF16, 40, 0, 1, 2, 128, 128) == 0  # a mask that does not say how long its tasks are
 
 
+@pytest.mark.parametrize("L,pieces", [(1560, 2), (1731, 3), (1800, 2)])
+def test_pieces_fit_the_engines(L, pieces):
+    """Workgroups go to an XCD's four engines in turn: 168 tiles (1731 tokens) in uneven pairs would
+    leave one engine six long and five short pieces, as long as the whole tiles."""
+    tiles, part = (L + 127) // 128 * 12, 4 * (2 * 128 * 128 + 256)
+    assert nat.fwd_split_bytes(F32, JVP, 1, 12, L, L, 128, 128) == tiles * pieces * part
+
+
 def test_argument_checks():
     with pytest.raises(ValueError):
         nat.fwd_split_bytes(BF16, JVP, 1, 2, 64, 64, 96, 96)
