@@ -315,12 +315,24 @@ def _eager_call(*ts) -> bool:
     """Whether this is an ordinary eager call, which runs the kernels straight from Python:
     nothing that watches or replaces operators (a compiler, torch.jit tracing, a dispatch or
     function mode such as selective checkpointing's or make_fx's, a functorch transform,
-    forward-mode AD, a tensor subclass, the profiler) needs to see the registered op. The op
-    costs about 7 us of host time per call beyond the call it wraps (15 us)."""
-    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
-                or torch._C._is_torch_function_mode_enabled() or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
-                or torch.autograd._profiler_enabled()) and _PLAIN_TENSORS.issuperset(map(type, ts))
+    forward-mode AD, a tensor subclass, the profiler) needs to see the registered op, and
+    every operand's memory holds its values. It does not for a meta tensor (the op answers
+    with shapes), for a zero tensor without memory and for a lazily negated view (the
+    dispatcher makes ordinary tensors of them), and for the batch of cotangents of
+    torch.autograd.grad(is_grads_batched=True) and vectorized jacobians, a torch.Tensor
+    outside functorch's stack whose data_ptr() raises (the dispatcher calls the op per
+    cotangent). The op costs about 7 us of host time per call beyond the call it wraps
+    (15 us), this check 3 us for the six operands of a JVP call."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._is_torch_function_mode_enabled() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+            or torch.autograd._profiler_enabled() or not _PLAIN_TENSORS.issuperset(map(type, ts))):
+        return False
+    ts = [t for t in ts if t is not None]
+    try:
+        return all(map(torch.Tensor.data_ptr, ts)) and not any(map(torch.Tensor.is_neg, ts))
+    except RuntimeError:
+        return False
 
 
 def _fwd_ws_bytes(dtype, mode, B, H, Lk, Dqk, Dv) -> int:
@@ -346,7 +358,7 @@ def _fwd_dense_ws_bytes(dtype, mode, B, H, Lk, Dqk, Dv) -> int:
 
 def _check_device(*ts):
     for t in ts:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(
                 "dmad_amd attention runs on the GPU only (HIP kernels); got a tensor on " + str(t.device)
             )
