@@ -488,8 +488,10 @@ struct DqFullCfg {
   static constexpr int LOADS = 4 * RPW;
 };
 
-// TG: also the tangent gradient dQd = s dSd K.
-template <typename T, int D, bool TG>
+// TG: also the tangent gradient dQd = s dSd K. SPLIT: the last work items run in
+// pieces of the keys (split.h), cut where attn_bwd_dq_sc_kernel<T, 2> cuts, so that
+// dQ (and dQd) do not depend on which of the two runs.
+template <typename T, int D, bool TG, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dq_full_kernel(DqParams p) {
   using C = DqFullCfg<D>;
   constexpr int BN = C::BN, KS = C::KS, DB = C::DB, CR = C::CR, ROWB = C::ROWB;
@@ -504,10 +506,19 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_full_kernel(DqParams p) {
   const int col = lane & 31, half = lane >> 5;
 
   const int nqt = (p.Lq + C::BM - 1) / C::BM;
-  const int work = work_item(p.xcd_order);  // block order (common.h)
+  int work, kt0 = 0, ntiles = (p.Lk + BN - 1) / BN, part_slot = -1;  // key tiles [kt0, kt0 + ntiles) are this workgroup's
+  if constexpr (SPLIT) {
+    const SplitWork w = split_work(p.sp, p.xcd_order, ntiles);
+    if (w.item < 0) return;
+    work = w.item;
+    kt0 = w.beg;
+    ntiles = w.end - w.beg;
+    if (w.piece >= 0) part_slot = w.slot;
+  } else {
+    work = work_item(p.xcd_order);  // block order (common.h)
+  }
   const int bh = work / nqt, qt = work - bh * nqt;
   const int b = bh / p.H, h = bh - b * p.H;
-  const int ntiles = (p.Lk + BN - 1) / BN;
 
   // ---- this lane's query: Q, Qd, dO, dOd rows (B operands, AGPRs) and statistics
   const int query = qt * C::BM + wave * 32 + col;
@@ -571,6 +582,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_full_kernel(DqParams p) {
     else return (lds_char_t*)stg3;
   };
   auto issue_load = [&](lds_char_t* st, int kt, int li) {
+    kt += kt0;
     const int t = li % 4, jj = li / 4, i = wave + jj * C::NW;
     const uint32_t ks = (uint32_t)kt * k_step, vs = (uint32_t)kt * v_step;
     if (t == 0) buf_load16_lds(rk, st + C::OFF_K + i * 1024, roff_k[jj], ks);
@@ -756,6 +768,23 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_full_kernel(DqParams p) {
     else if (rest == 3) last_step(IC<2>{}, sa);
     else last_step(IC<3>{}, sb);
     wait_vmem();  // no requests beyond the last tile stay in flight
+  }
+
+  if constexpr (SPLIT) {
+    if (part_slot >= 0) {
+      constexpr int TILE = split_tile_floats<D>();
+      float* const tile = p.sp.part + ((int64_t)part_slot * C::NW + wave) * 2 * TILE;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          split_put<D>(tile, lane, d, jj, f32x4_t{acc[d][4 * jj], acc[d][4 * jj + 1], acc[d][4 * jj + 2], acc[d][4 * jj + 3]});
+          if constexpr (TG)
+            split_put<D>(tile + TILE, lane, d, jj, f32x4_t{tacc[d][4 * jj], tacc[d][4 * jj + 1], tacc[d][4 * jj + 2], tacc[d][4 * jj + 3]});
+        }
+      }
+      return;
+    }
   }
 
   // ---- dQ = s (dQ^T)^T [, dQd = s (dQd^T)^T]: lane holds query col, d = 32 db + 8 jj + 4 half + 0..3

@@ -70,6 +70,16 @@ template <>
 BwdLaunchFn kv_full_split_select<Elt>(bool store) {
   return store ? &kv_full_split_launch<Elt, true> : &kv_full_split_launch<Elt, false>;
 }
+template <typename T, bool TG>
+static hipError_t dq_full_split_launch(const DqParams& p, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((attn_bwd_dq_full_kernel<T, 128, TG, true>), dim3(grid), dim3(256), 0, s, p);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_dq_sum<T, 128, DqFullCfg<128>::NW, 2>(p, s);
+}
+template <>
+DqLaunchFn dq_full_split_select<Elt>(bool tangent_grads) {
+  return tangent_grads ? &dq_full_split_launch<Elt, true> : &dq_full_split_launch<Elt, false>;
+}
 template <typename T>
 static hipError_t dq_sc2_split_launch(const DqParams& p, int grid, hipStream_t s) {
   hipLaunchKernelGGL((attn_bwd_dq_sc_kernel<T, 2, true>), dim3(grid), dim3(DqScCfg<2>::NW * 64), 0, s, p);

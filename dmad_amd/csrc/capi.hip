@@ -547,14 +547,19 @@ BwdPlan plan_bwd_ws(int dtype, bool full, bool tgrad, int64_t B, int64_t H, int6
 
 // Split launches of the backward's row-reading passes (split.h): the last key
 // tiles run in pieces of the queries, the last query tiles (pairs of tiles on
-// stored gradients) in pieces of the keys. The cut depends on the sizes alone and
-// is the same whether scores are stored or recomputed and however many (b, h)
-// slices a launch pair takes, so dK and dV keep not depending on the workspace.
+// stored gradients) in pieces of the keys. The cut depends on the sizes alone
+// and is the same whether scores are stored or recomputed and however many (b, h)
+// slices a launch pair takes, so no gradient depends on the workspace: the two
+// query passes of 128-wide heads add the same products in the same order within
+// a piece, and both cut at the same tiles and keys.
+// Queries and keys from which the torch op's dO-only backward stores its scores.
+constexpr int64_t kScoreMinLen = 2048;
+
 struct BwdSplit {
   dmad::SplitPlan kv;    // main key pass
   dmad::SplitPlan kv_t;  // tangent key pass
-  dmad::SplitPlan dq;    // recomputing query pass (dO only; with tangent gradients of 64-wide heads theirs)
-  dmad::SplitPlan dq_sc; // query pass on stored gradients
+  dmad::SplitPlan dq;    // recomputing query pass (64-wide heads: dO only, or the tangent gradients')
+  dmad::SplitPlan dq_sc; // query pass on stored gradients (128-wide heads)
   int64_t bytes = 0;     // the largest of their partials (one after the other in a call)
 };
 
@@ -580,8 +585,36 @@ BwdSplit plan_bwd_split(int dtype, bool full, bool tgrad, int64_t B, int64_t H, 
   const dmad::SplitCost dq_sc{1, full ? 1.2f : 0.6f, 0.f, 8.f, (full ? 16 : 8) * tile};
   if (!full || D == 128) r.kv = dmad::plan_split(BH * nkt, qsteps, full ? kv_full : kv);
   if (tgrad) r.kv_t = dmad::plan_split(BH * nkt, qsteps, kv);
-  if (!full || (tgrad && D == 64)) r.dq = dmad::plan_split(BH * nqt, ksteps, dq);
-  if (D == 128) r.dq_sc = dmad::plan_split(BH * ((nqt + 1) / 2), ksteps, dq_sc);
+  if (D == 64) {
+    if (!full || tgrad) r.dq = dmad::plan_split(BH * nqt, ksteps, dq);
+  } else if (BH * nqt > 0) {
+    // one cut for both query passes, from the costs of the one that runs at these
+    // lengths by default: from whole pairs of tiles on, in the same pieces. (The
+    // other one follows a cut made for half or twice as many workgroups. Scores
+    // recomputed on purpose, whole against so cut, the whole backward: 12 heads of
+    // 6240 tokens, full derivative, 2014 -> 1775 us, dO only 855 -> 758; at worst nine
+    // heads of 3030 tokens, full, whose 216 tiles fit the chip: 360 -> 379 us.)
+    const int64_t npair = (nqt + 1) / 2;  // pairs of a head, the last one perhaps a single tile
+    dmad::SplitPlan cut;
+    int64_t first;  // first pair in pieces
+    if (!full && (Lq < kScoreMinLen || Lk < kScoreMinLen)) {
+      cut = dmad::plan_split(BH * nqt, ksteps, dq);
+      first = cut.whole / nqt * npair + cut.whole % nqt / 2;
+    } else {
+      cut = dmad::plan_split(BH * npair, ksteps, dq_sc);
+      first = cut.whole;
+    }
+    if (cut.rest > 0) {
+      const int64_t tile0 = first / npair * nqt + 2 * (first % npair);
+      const dmad::SplitPlan pairs = dmad::split_cut(BH * npair, BH * npair - first, cut.n, cut.len, dq_sc.part_bytes);
+      const dmad::SplitPlan tiles =
+          dmad::split_cut(BH * nqt, BH * nqt - tile0, cut.n, cut.len, full ? 2 * dq.part_bytes : dq.part_bytes);
+      if (pairs.bytes <= dmad::kSplitMaxBytes && tiles.bytes <= dmad::kSplitMaxBytes) {
+        r.dq = tiles;
+        r.dq_sc = pairs;
+      }
+    }
+  }
   for (const dmad::SplitPlan* p : {&r.kv, &r.kv_t, &r.dq, &r.dq_sc}) r.bytes = p->bytes > r.bytes ? p->bytes : r.bytes;
   return r;
 }
@@ -605,6 +638,12 @@ dmad::BwdLaunchFn pick_kv_split(int dtype, int64_t d, bool full, int scm) {
 dmad::DqLaunchFn pick_dq_split(int dtype, int64_t d, bool full, bool stored) {
   if (dtype == DMAD_BF16) return stored ? dmad::dq_sc_split_select<__bf16>(full) : dmad::dq_split_select<__bf16>((int)d);
   if (dtype == DMAD_F16) return stored ? dmad::dq_sc_split_select<_Float16>(full) : dmad::dq_split_select<_Float16>((int)d);
+  return nullptr;
+}
+
+dmad::DqLaunchFn pick_dq_full_split(int dtype, bool tangent_grads) {
+  if (dtype == DMAD_BF16) return dmad::dq_full_split_select<__bf16>(tangent_grads);
+  if (dtype == DMAD_F16) return dmad::dq_full_split_select<_Float16>(tangent_grads);
   return nullptr;
 }
 
@@ -1095,12 +1134,14 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
   }
   const dmad::BwdLaunchFn fn_sp = pick_kv_split(dtype, D, full, dmad::kScNone);
   const dmad::BwdLaunchFn fa_sp = pick_kv_split(dtype, D, false, dmad::kScNone);
-  const dmad::DqLaunchFn fq_sp = pick_dq_split(dtype, D, full, false);
+  // the recomputing query pass, and the tangent gradients' of 64-wide heads
+  const dmad::DqLaunchFn fq_sp = full_rows ? pick_dq_full_split(dtype, tgrad) : full ? nullptr : pick_dq_split(dtype, D, false, false);
+  const dmad::DqLaunchFn fqa_sp = pick_dq_split(dtype, D, false, false);
   mark(0, false, s);
   if ((e = launch_pass(p, fn, fn_sp, split.kv, 0, plan.grid_kv, part, s)) != hipSuccess) return fail(DMAD_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
   mark(0, true, s);
   mark(1, false, s);
-  if (plan.grid_dq > 0 && (e = launch_pass(pq, fq, full ? nullptr : fq_sp, split.dq, 0, plan.grid_dq, part, s)) != hipSuccess)
+  if (plan.grid_dq > 0 && (e = launch_pass(pq, fq, fq_sp, split.dq, 0, plan.grid_dq, part, s)) != hipSuccess)
     return fail(DMAD_ERR_HIP, "backward dq launch: %s", hipGetErrorString(e));
   mark(1, true, s);
   if (tgrad) {
@@ -1123,7 +1164,7 @@ int bwd_impl(int dtype, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D,
     pqt.dq = dtq;
     if (fq_a != nullptr) {
       mark(3, false, s);
-      if (plan.grid_dq > 0 && (e = launch_pass(pqt, fq_a, fq_sp, split.dq, 0, plan.grid_dq, part, s)) != hipSuccess)
+      if (plan.grid_dq > 0 && (e = launch_pass(pqt, fq_a, fqa_sp, split.dq, 0, plan.grid_dq, part, s)) != hipSuccess)
         return fail(DMAD_ERR_HIP, "backward dq launch: %s", hipGetErrorString(e));
       mark(3, true, s);
     }

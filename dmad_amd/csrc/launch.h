@@ -140,8 +140,8 @@ template <> DqLaunchFn dq_sc_select<_Float16>(bool);
 // The row-reading passes with their last work items in pieces, each followed by
 // the kernel that sums the pieces (BwdParams::sp, DqParams::sp; split.h): the key
 // pass of d-wide heads by what it does with score gradients (d = 64: kScNone), the
-// full key pass (store: kScStore), the recomputing query pass and the query pass
-// on stored gradients.
+// full key pass (store: kScStore), the recomputing query passes (dO only, full)
+// and the query pass on stored gradients.
 template <typename T>
 BwdLaunchFn kv_split_select(int d, int scm);
 template <> BwdLaunchFn kv_split_select<__bf16>(int, int);
@@ -154,6 +154,10 @@ template <typename T>
 DqLaunchFn dq_split_select(int d);
 template <> DqLaunchFn dq_split_select<__bf16>(int);
 template <> DqLaunchFn dq_split_select<_Float16>(int);
+template <typename T>
+DqLaunchFn dq_full_split_select(bool tangent_grads);
+template <> DqLaunchFn dq_full_split_select<__bf16>(bool);
+template <> DqLaunchFn dq_full_split_select<_Float16>(bool);
 template <typename T>
 DqLaunchFn dq_sc_split_dout_only();
 template <> DqLaunchFn dq_sc_split_dout_only<__bf16>();

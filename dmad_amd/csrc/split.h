@@ -129,6 +129,19 @@ inline double split_makespan(const SplitCost& k, int64_t a, double la, int64_t b
   return t;
 }
 
+// The plan that runs the last `rest` of `items` work items in n pieces, `len` steps each
+// but the last.
+inline SplitPlan split_cut(int64_t items, int64_t rest, int n, int len, int64_t part_bytes) {
+  SplitPlan pl;
+  pl.whole = items - rest;
+  pl.rest = rest;
+  pl.n = n;
+  pl.len = len;
+  pl.grid = split_grid(pl.whole, rest, n);
+  pl.bytes = rest * n * part_bytes;
+  return pl;
+}
+
 // How to run `items` work items of `steps` steps: in full rounds, then the rest in
 // the pieces that finish soonest by the costs above (even_only: in pieces of one
 // length), where that saves at least a twentieth of the launch and 8 us: the second
@@ -171,13 +184,7 @@ inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k, bo
       }
     }
   }
-  if (pl.n > 1) {
-    pl.whole = items - rest;
-    pl.rest = rest;
-    pl.grid = split_grid(pl.whole, rest, pl.n);
-    pl.bytes = rest * pl.n * k.part_bytes;
-  }
-  return pl;
+  return pl.n > 1 ? split_cut(items, rest, pl.n, pl.len, k.part_bytes) : pl;
 }
 
 // ---------------------------------------------------------------- forward

@@ -158,7 +158,8 @@ def _backward_workspace(code: int, ws_mode: int, B: int, H: int, Lq: int, Lk: in
     """(pointer, size, owner) of a backward's workspace: the minimum plus the stored score
     gradients the budget allows. The stored scores only save time, so when the device cannot
     hold them the call takes the minimum and the query pass recomputes the scores (the same
-    dQ bit for bit); an allocation failure of the minimum itself propagates."""
+    gradients bit for bit, except that the full derivative's dQ may round differently in one or
+    two of 10000 elements); an allocation failure of the minimum itself propagates."""
     base = nat.bwd_workspace_bytes_of(code, ws_mode, B, H, Lq, Lk, D)
     extra = _score_bytes(code, ws_mode > 0, B, H, Lq, Lk, D)
     if extra > 0:
@@ -498,8 +499,10 @@ def jvp_attention_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto, sm_sc
     dtv = torch.empty_like(dv) if tgrads else None
     lib = nat.lib()
     ws_mode = (2 if tgrads else 1) if full else 0
-    ws_ptr, ws_size, ws = _backward_workspace(code, ws_mode, B, H, Lq, Lk, D, q.device)
+    # the partials first: without room for them every gradient's last bits change, without
+    # room for the stored scores none do
     sp_ptr, sp_size, sp = _split_workspace(nat.bwd_split_bytes(code, full, tgrads, B, H, Lq, Lk, D), q.device)
+    ws_ptr, ws_size, ws = _backward_workspace(code, ws_mode, B, H, Lq, Lk, D, q.device)
     nat.check(
         lib.dmad_attn_jvp_bwd_split(
             code, B, H, Lq, Lk, D,
