@@ -398,9 +398,10 @@ __global__ __launch_bounds__(f32_fwd_wide(MODE, DQK) ? 256 : 512) void attn_f32_
         if constexpr (C::JVP) *(f32x4_t*)(tile + P::TILE + (d * 64 + lane) * 4) = cacc[d] * keep_l;
       }
       if (g == 0) {
-        float* const st = part + P::STATS + wave * 32 + col;
-        st[0] = m_i + __builtin_log2f(l);
-        if constexpr (C::JVP) st[16] = l == 0.f ? 0.f : mu;
+        float* const st = part + P::STATS + wave * P::NS * 16 + col;
+        st[0] = m_i;
+        st[16] = l;
+        if constexpr (C::JVP) st[32] = l == 0.f ? 0.f : mu;
       }
       return;
     }

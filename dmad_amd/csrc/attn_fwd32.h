@@ -136,7 +136,7 @@ __device__ __forceinline__ void stage_store(const lds_char_t* region, int k, int
 //
 // SPLIT (64- and 128-wide heads): the last work items of the grid run in pieces of
 // their key range, or of their task's key tiles (split.h); a piece sees its keys as the whole
-// sequence and writes O~ / l, C~ / l, its logsumexp and mu as fp32 partials.
+// sequence and writes O~ / l, C~ / l, its maximum, l and mu as fp32 partials.
 template <typename T, int MODE, bool MAGI = false, int DH = 128, bool SPLIT = false>
 __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2) : 1) void attn_fwd32_kernel(
     FwdParams p) {
@@ -719,9 +719,10 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
         if constexpr (kAccAgpr) __builtin_amdgcn_sched_barrier(0);
       }
       if (half == 0) {
-        float* const st = part + P::STATS + wave * 64 + col;
-        st[0] = exp_base<T>(m_i) + __builtin_log2f(l);
-        if constexpr (C::JVP) st[32] = l == 0.f ? 0.f : mu;
+        float* const st = part + P::STATS + wave * P::NS * 32 + col;
+        st[0] = exp_base<T>(m_i);
+        st[32] = l;
+        if constexpr (C::JVP) st[64] = l == 0.f ? 0.f : mu;
       }
       return;
     }

@@ -288,7 +288,7 @@ dmad::SplitCost fwd_split_cost(int mode, int64_t D) {
 // tiles in two uneven pieces each, 310 -> 219 us at 64 and 598 -> 417 us at 128 wide.
 dmad::SplitCost f32_fwd_split_cost(int mode, int64_t D) {
   const bool jvp = mode != DMAD_FWD_PLAIN;
-  return {1, (jvp ? 0.1f : 0.035f) * (float)D, 0.f, 6.f, (int)((128 * D * (jvp ? 2 : 1) + 256) * 4)};
+  return {1, (jvp ? 0.1f : 0.035f) * (float)D, 0.f, 6.f, (int)((128 * D * (jvp ? 2 : 1) + (jvp ? 384 : 256)) * 4)};
 }
 
 // The split of a dense forward's last query tiles over their keys. Both JVP

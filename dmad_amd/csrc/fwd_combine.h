@@ -34,7 +34,7 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdParams p) {
   const int query = row0 + wave * ROWS + col;
   auto empty = [&](int i) { return MAGI && magi_piece(ntiles, i, p.sp.n) == magi_piece(ntiles, i + 1, p.sp.n); };
   const float* part = p.sp.part + (int64_t)item * p.sp.n * P::FLOATS;
-  const float* st = part + P::STATS + wave * 2 * ROWS + col;
+  const float* st = part + P::STATS + wave * P::NS * ROWS + col;
   // pieces are taken U at a time with all of their loads in flight together (the
   // partials come from other XCDs' workgroups, about a microsecond away); past
   // the last piece the last one is read again and left out
@@ -55,12 +55,14 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdParams p) {
   for (int g = 0; g < NG; ++g) o[g] = c[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int i = 0; i < n; i += U) {
     f32x4_t ov[U][NG], cv[U][NG];
-    float lse2[U], mus[U];
+    float ms[U], ls[U], mus[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const float* pi = part + (int64_t)min(i + u, n - 1) * P::FLOATS;
-      lse2[u] = pi[P::STATS + wave * 2 * ROWS + col];
-      if constexpr (JVP) mus[u] = pi[P::STATS + wave * 2 * ROWS + ROWS + col];
+      const float* si = st + (pi - part);
+      ms[u] = si[0];
+      ls[u] = si[ROWS];
+      if constexpr (JVP) mus[u] = si[2 * ROWS];
       const float* tile = pi + wave * P::NT * P::TILE;
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
@@ -74,7 +76,7 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdParams p) {
     for (int u = 0; u < U; ++u) {
       if (i + u >= n) break;
       if (empty(i + u)) continue;
-      const float wi = fast_exp2(lse2[u] - m);
+      const float wi = fast_exp2(ms[u] - m) * ls[u];
       w += wi;
       if constexpr (JVP) mu += wi * mus[u];
 #pragma unroll

@@ -189,8 +189,10 @@ inline SplitPlan plan_split(int64_t items, int64_t steps, const SplitCost& k, bo
 
 // ---------------------------------------------------------------- forward
 // Partial block of the forward, 128 queries: per wave [O (, C)][ROWS x D], then per
-// wave [lse2, mu][ROWS]. O = O~ / l and C = C~ / l of the piece's keys, lse2 its
-// log2-domain logsumexp. ROWS = 32: tiles as above. ROWS = 16 (fp32 operands): the
+// wave [m, l (, mu)][ROWS]: l the sum of exp2(score - m) over the piece's keys,
+// O = O~ / l and C = C~ / l. A piece weighs exp2(m) l; m + log2(l) in one float
+// would lose l beside scores of a large common value (2^24 and more: all of it).
+// ROWS = 32: tiles as above. ROWS = 16 (fp32 operands): the
 // 16x16 layout (lane: row lane % 16, columns 16 d + 4 (lane / 16) + 0..3), again
 // 16 bytes per lane and d.
 template <int D, bool JVP, int ROWS = 32>
@@ -199,7 +201,8 @@ struct FwdPart {
   static constexpr int NT = JVP ? 2 : 1;
   static constexpr int TILE = ROWS * D;
   static constexpr int STATS = WAVES * NT * TILE;
-  static constexpr int FLOATS = STATS + WAVES * 2 * ROWS;
+  static constexpr int NS = JVP ? 3 : 2;
+  static constexpr int FLOATS = STATS + WAVES * NS * ROWS;
 };
 
 // ---------------------------------------------------------------- backward

@@ -104,6 +104,33 @@ def test_split_forward_with_masked_pieces(gpu, D, dtype):
     assert float((lse.cpu().double() - rlse).abs().max()) <= 2e-3
 
 
+@pytest.mark.parametrize("mode", ["plain", "jvp"])
+@pytest.mark.parametrize("offset", [-2.0 ** 30, 2.0 ** 17])
+@pytest.mark.parametrize("Lk,D,dtype", [(2010, 64, torch.bfloat16), (2010, 128, torch.bfloat16), (900, 64, torch.float32)])
+def test_split_forward_beside_a_large_common_score(gpu, mode, offset, Lk, D, dtype):
+    """Rows all of whose scores are one large value (a caller's mask as a feature of K, in rows that
+    it masks throughout): a piece weighs by the number of its keys, which differ."""
+    from dmad_amd import _native as nat
+    from dmad_amd.jvp_attention import jvp_attention_forward
+
+    print(f"case common score {mode} {offset} {Lk} {D} {dtype}", flush=True)
+    nmode = nat.DMAD_FWD_PLAIN if mode == "plain" else nat.DMAD_FWD_JVP
+    assert nat.fwd_split_bytes(nat.dtype_code(dtype), nmode, 1, 2, 200, Lk, D, D) > 0
+    q, k, v, tq, tk, tv = _draw(gpu, 5, 1, 2, 200, Lk, D, dtype)
+    v += (torch.arange(Lk, device=gpu) / Lk).to(dtype)[None, None, :, None]  # uneven over the keys
+    q.zero_()
+    q[..., 0] = 1.0
+    tq[..., 0] = 0.0
+    k[..., 0] = 0.0
+    xs = (q, k, v, tq, tk, tv)
+    ref = orc.jvp_closed_form(*(t.cpu().double() for t in xs), sm_scale=1.0)  # a common score changes nothing
+    k[..., 0] = offset
+    o, to, _, mu = jvp_attention_forward(*(xs if mode == "jvp" else (q, k, v, None, None, None)), 1.0)
+    assert orc.rel_l2(o.cpu(), ref[0]) <= (1e-2 if dtype == torch.bfloat16 else 1e-5)
+    if mode == "jvp":
+        assert orc.rel_l2(to.cpu(), ref[1]) <= 1e-2 and orc.rel_l2(mu.cpu(), ref[3]) <= 1e-2
+
+
 BWD = [
     # B, H, Lq, Lk, D, full derivative with tangent gradients
     (1, 2, 2300, 2300, 64, False),

@@ -59,7 +59,7 @@ def test_full_rounds_and_other_head_dims_stay_whole():
 def test_pieces_fit_the_engines(L, pieces):
     """Workgroups go to an XCD's four engines in turn: 168 tiles (1731 tokens) in uneven pairs would
     leave one engine six long and five short pieces, as long as the whole tiles."""
-    tiles, part = (L + 127) // 128 * 12, 4 * (2 * 128 * 128 + 256)
+    tiles, part = (L + 127) // 128 * 12, 4 * (2 * 128 * 128 + 3 * 128)  # O, C and three statistics of 128 rows
     assert nat.fwd_split_bytes(F32, JVP, 1, 12, L, L, 128, 128) == tiles * pieces * part
 
 
