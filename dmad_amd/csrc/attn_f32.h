@@ -258,8 +258,8 @@ __global__ __launch_bounds__(f32_fwd_wide(MODE, DQK) ? 256 : 512) void attn_f32_
     oacc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     cacc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  // (a piece starts from a finite maximum: attn_fwd32_kernel)
-  float m_i = SPLIT ? -3.0e38f : -__builtin_inff(), l_i = 0.f, r_i = 0.f;
+  // (a piece starts from the lowest finite maximum: attn_fwd32_kernel)
+  float m_i = SPLIT ? kLowest : -__builtin_inff(), l_i = 0.f, r_i = 0.f;
 
   auto fetch = [&](int start) {
     fetch_k(start);

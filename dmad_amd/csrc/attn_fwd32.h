@@ -462,9 +462,9 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   // 16 (v >> 3) + 8 half + (v & 7); P~, H~ are packed as the B operands of the
   // two 16-key chunks.
   constexpr int NMICRO = 18;
-  // a piece starts from a finite maximum, so that a row all of whose keys in it
-  // score -inf has l = 0 there rather than NaN
-  float m_i = SPLIT ? -3.0e38f : -__builtin_inff(), l_i = 0.f, r_i = 0.f;
+  // a piece starts from the lowest finite maximum, so that a row all of whose keys
+  // in it score -inf has l = 0 there rather than NaN; no finite score lies below it
+  float m_i = SPLIT ? kLowest : -__builtin_inff(), l_i = 0.f, r_i = 0.f;
   struct Soft {
     float mx, alpha, neg_m, ls, rs, pv;
     float hv;

@@ -157,6 +157,8 @@ __device__ __forceinline__ void mfma_acc_drain(f32x16_t (&... acc)[N]) {
   (redefine(acc), ...);
 }
 
+constexpr float kLowest = -3.402823466e+38f;  // the lowest finite float
+
 // 16x16x32 layouts: A (16 x 32): lane l holds row l%16, k = 8*(l/16) + e;
 // B (32 x 16): lane l holds col l%16, k = 8*(l/16) + e;
 // C (16 x 16): lane l holds col l%16, rows 4*(l/16) + v, v = 0..3.

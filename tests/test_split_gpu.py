@@ -131,6 +131,38 @@ def test_split_forward_beside_a_large_common_score(gpu, mode, offset, Lk, D, dty
         assert orc.rel_l2(to.cpu(), ref[1]) <= 1e-2 and orc.rel_l2(mu.cpu(), ref[3]) <= 1e-2
 
 
+@pytest.mark.parametrize("mode", ["plain", "jvp"])
+@pytest.mark.parametrize("B,H,Lq,Lk,D,dtype", [
+    (1, 2, 200, 2000, 64, torch.bfloat16), (1, 2, 200, 2000, 128, torch.bfloat16), (1, 2, 200, 900, 64, torch.float32),
+    (1, 21, 3200, 3000, 128, torch.bfloat16)])  # the last one: full rounds of whole tiles, too
+@pytest.mark.parametrize("whole", [False, True])
+def test_split_forward_at_the_lowest_scores(gpu, monkeypatch, whole, mode, B, H, Lq, Lk, D, dtype):
+    """Rows all of whose scores are bf16's lowest value (a caller's mask as a feature of K): equal
+    scores, finite ones, so the softmax is uniform, as in a launch that does not split."""
+    from dmad_amd import _native as nat
+    from dmad_amd.jvp_attention import jvp_attention_forward
+
+    print(f"case lowest scores {mode} {B} {H} {Lq} {Lk} {D} {dtype}", flush=True)
+    nmode = nat.DMAD_FWD_PLAIN if mode == "plain" else nat.DMAD_FWD_JVP
+    assert nat.fwd_split_bytes(nat.dtype_code(dtype), nmode, B, H, Lq, Lk, D, D) > 0
+    q, k, v, tq, tk, tv = _draw(gpu, 5, B, H, Lq, Lk, D, dtype)
+    if whole:
+        monkeypatch.setattr(nat, "fwd_split_bytes", lambda *a: 0)
+    q.zero_()
+    q[..., 0] = 1.0
+    k[..., 0] = torch.finfo(torch.bfloat16).min
+    tq[..., 0] = 0.0
+    scale = 0.6931471824645996  # times log2(e) rounds to 1: the scores in the log2 domain are as given
+    xs = (q, k, v, tq, tk, tv) if mode == "jvp" else (q, k, v, None, None, None)
+    o, to, lse, mu = (None if t is None else t[:, -1:].cpu() for t in jvp_attention_forward(*xs, scale))
+    assert bool((lse == torch.finfo(torch.bfloat16).min * 0.6931471805599453).all())
+    k[..., 0] = 0.0  # equal scores for the oracle (exp(S - LSE) in float64 would lose log(Lk) beside 1e38)
+    ref = orc.jvp_closed_form(*(t[:, -1:].cpu().double() for t in (q, k, v, tq, tk, tv)), sm_scale=scale)
+    assert orc.rel_l2(o, ref[0]) <= 1e-2
+    if mode == "jvp":
+        assert orc.rel_l2(to, ref[1]) <= 1e-2 and orc.rel_l2(mu, ref[3]) <= 1e-2
+
+
 BWD = [
     # B, H, Lq, Lk, D, full derivative with tangent gradients
     (1, 2, 2300, 2300, 64, False),
