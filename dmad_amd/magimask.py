@@ -217,13 +217,17 @@ def group_q_ranges_csr(q_ranges: torch.Tensor, k_ranges: torch.Tensor) -> Tuple[
     """Runs of equal consecutive query ranges -> (q_unique [G,2], k_flat [R,2], qk_map [G+1])
     (train/wan/rcm/utils/magimask.py:187-213)."""
     assert q_ranges.ndim == 2 and q_ranges.shape[1] == 2 and k_ranges.shape == q_ranges.shape
-    qs = _host(q_ranges)
-    starts = [0] + [i for i in range(1, len(qs)) if (qs[i] != qs[i - 1]).any()]
-    qk_map = np.asarray(starts + [len(qs)], dtype=np.int64)
+    starts, qk_map = _groups(_host(q_ranges))
     dev = q_ranges.device
-    return (q_ranges.contiguous()[torch.as_tensor(starts, dtype=torch.long, device=dev)].contiguous(),
+    return (q_ranges.contiguous()[torch.as_tensor(starts, device=dev)].contiguous(),
             k_ranges.contiguous(),
             torch.tensor(qk_map, device=dev, dtype=torch.int32))
+
+
+def _groups(qs: np.ndarray) -> Tuple[np.ndarray, np.ndarray]:
+    """group_q_ranges_csr on the host: (first row of each run, qk_map)."""
+    starts = np.flatnonzero(np.append(True, (qs[1:] != qs[:-1]).any(axis=1)))
+    return starts, np.append(starts, len(qs))
 
 
 def _tasks(qu: np.ndarray, Q_real: int, block_m: int) -> Tuple[np.ndarray, np.ndarray]:
@@ -267,20 +271,20 @@ def prepare_magi_csr_and_tasks(q_ranges: torch.Tensor, k_ranges: torch.Tensor, Q
     """Merge, group, check that the query groups partition [0, Q_real), build tasks
     (train/wan/rcm/utils/magimask.py:265-283). BLOCK_M defaults to the kernels' 128."""
     rows, dev = _merged(q_ranges, k_ranges, KV_real), q_ranges.device
-    new = np.flatnonzero(np.append(True, (rows[1:, :2] != rows[:-1, :2]).any(axis=1))) if len(rows) else np.zeros(0, int)
-    qu = rows[new, :2]
+    starts, qk_map = _groups(rows[:, :2])
+    qu = rows[starts, :2]
     assert len(qu) > 0 and qu[0, 0] == 0 and qu[-1, 1] == Q_real, \
         f"the query groups must start at row 0 and end at row {Q_real} (Q_real)"
     for i in range(len(qu) - 1):
         assert qu[i, 1] == qu[i + 1, 0], \
             f"query groups {i} and {i + 1} do not meet: {qu[i].tolist()} then {qu[i + 1].tolist()}"
     task_group, task_qtile = _tasks(qu, Q_real, BLOCK_M)
-    most = np.add.reduceat((rows[:, 3] + 31) // 32 - rows[:, 2] // 32, new).max()
+    most = np.add.reduceat((rows[:, 3] + 31) // 32 - rows[:, 2] // 32, starts).max()
 
     def table(x):
         return torch.tensor(x, device=dev, dtype=torch.int32)
 
-    return MagiMask(q_unique=table(qu), k_flat=table(rows[:, 2:]), qk_map=table(np.append(new, len(rows))),
+    return MagiMask(q_unique=table(qu), k_flat=table(rows[:, 2:]), qk_map=table(qk_map),
                     task_group=table(task_group), task_qtile=table(task_qtile), G=len(qu), T=len(task_group),
                     BLOCK_M=int(BLOCK_M), key_tiles=int(most))
 

@@ -292,3 +292,31 @@ def test_dispatcher_decision_and_cache():
     assert mod.get_magi_mask(spec, 48, 48, "cpu") is not a
     mod.clear_cache()
     assert mod.get_magi_mask(spec, 80, 80, "cpu") is not a
+
+
+def test_prepared_tables_are_those_of_the_single_steps():
+    """prepare_magi_csr_and_tasks builds its tables on the host: the same as merging, grouping and
+    building tasks one by one, and key_tiles is the longest walk over a group's key ranges."""
+    import random
+
+    from dmad_amd import magimask as mm
+
+    r = random.Random(3)
+    for _ in range(50):
+        L, cuts = r.randint(1, 900), set()
+        while len(cuts) < r.randint(0, 5) and L > 1:
+            cuts.add(r.randint(1, L - 1))
+        edges = [0, *sorted(cuts), L]
+        rows = [(a, b, *sorted(r.sample(range(0, 1100), 2))) for a, b in zip(edges, edges[1:]) for _ in range(r.randint(1, 4))]
+        rows += [(a, b, 0, 1) for a, b in zip(edges, edges[1:])]  # no group without keys
+        r.shuffle(rows)
+        qr, kr = (torch.tensor([x[i:i + 2] for x in rows], dtype=torch.int32) for i in (0, 2))
+        m = mm.prepare_magi_csr_and_tasks(qr, kr, Q_real=L, KV_real=1000)
+        q2, k2 = mm.merge_k_ranges(qr, kr, KV_real=1000)
+        qu, kf, qm = mm.group_q_ranges_csr(q2, k2)
+        tg, tq = mm.build_qtile_tasks(qu, L, mm.KERNEL_BLOCK_M)
+        for a, b in zip((m.q_unique, m.k_flat, m.qk_map, m.task_group, m.task_qtile), (qu, kf, qm, tg, tq)):
+            assert torch.equal(a, b) and a.dtype == b.dtype == torch.int32
+        assert (m.G, m.T) == (len(qu), len(tg))
+        walks = [sum(len({key // 32 for key in range(a, b)}) for a, b in kf[qm[i]:qm[i + 1]].tolist()) for i in range(m.G)]
+        assert m.key_tiles == max(walks)
