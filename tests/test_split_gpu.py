@@ -104,6 +104,31 @@ def test_split_forward_with_masked_pieces(gpu, D, dtype):
     assert float((lse.cpu().double() - rlse).abs().max()) <= 2e-3
 
 
+@pytest.mark.parametrize("mode", ["jvp", "q"])
+@pytest.mark.parametrize("Lk,live,D,dtype", [(2000, 700, 64, torch.bfloat16), (2000, 700, 128, torch.bfloat16),
+                                             (900, 300, 64, torch.float32)])
+def test_split_jvp_with_masked_pieces(gpu, mode, Lk, live, D, dtype):
+    """The same with tangents: scores that overflow to -inf, as a caller's finite mask feature can
+    (an infinite one has no finite tangent)."""
+    from dmad_amd import _native as nat
+    from dmad_amd.jvp_attention import jvp_attention_forward
+
+    print(f"case masked jvp pieces {mode} {Lk} {D} {dtype}", flush=True)
+    assert nat.fwd_split_bytes(nat.dtype_code(dtype), nat.DMAD_FWD_JVP, 1, 2, 200, Lk, D, D) > 0
+    q, k, v, tq, tk, tv = _draw(gpu, 3, 1, 2, 200, Lk, D, dtype)
+    for t in (k, tq, tk):
+        t[..., 0] = 0.0
+    q[..., 0] = 1e20
+    k[:, :, live:, 0] = -1e30
+    if mode == "q":
+        tk, tv = torch.zeros_like(k), torch.zeros_like(v)
+    got = jvp_attention_forward(q, k, v, tq, *((tk, tv) if mode == "jvp" else (None, None)), D ** -0.5)
+    ref = orc.jvp_closed_form(*(t.cpu().double()[:, :, :live] if t.shape[2] == Lk else t.cpu().double()
+                                for t in (q, k, v, tq, tk, tv)))
+    for name, a, r in zip(("o", "to", "lse", "mu"), got, ref):
+        assert orc.rel_l2(a.cpu(), r) <= (1e-2 if dtype == torch.bfloat16 else 1e-5), name
+
+
 @pytest.mark.parametrize("mode", ["plain", "jvp"])
 @pytest.mark.parametrize("offset", [-2.0 ** 30, 2.0 ** 17])
 @pytest.mark.parametrize("Lk,D,dtype", [(2010, 64, torch.bfloat16), (2010, 128, torch.bfloat16), (900, 64, torch.float32)])
@@ -256,3 +281,54 @@ def test_split_block_sparse_forward(gpu, hint, kv_tangents, D, dtype):
         keep = torch.cat([torch.arange(330), torch.arange(400, 650)])
         _no_worse(name, a[:, :, keep], w[:, :, keep], r[:, :, keep])
         assert torch.equal(a[:, :, 330:400], w[:, :, 330:400]), name  # no keys: zeros, LSE -inf
+
+
+@pytest.mark.parametrize("B,H,D,dtype", [(1, 2, 128, torch.bfloat16), (2, 2, 128, torch.float16), (1, 5, 128, torch.bfloat16),
+                                         (1, 4, 64, torch.bfloat16), (3, 2, 64, torch.float16)])
+@pytest.mark.parametrize("kv_tangents", [True, False])
+def test_split_block_sparse_forward_after_full_rounds(gpu, kv_tangents, B, H, D, dtype):
+    """Masks of more tasks than one round takes: whole tasks first (dealt over the chip from the last
+    one down up to four heads, contiguous per XCD beyond), then the rest in pieces."""
+    import dataclasses
+
+    from dmad_amd import _native as nat
+    from dmad_amd import magimask as mm
+    from dmad_amd.jvp_attention import jvp_attention_forward_magi
+    from oracle import magi as om
+
+    slots = 256 if D == 128 else 512  # workgroups of a round
+    groups, Lk = 8, 1700 if D == 128 else 3300
+    tiles = slots // (B * H) + 3  # query tiles of a head: a round and a few
+    Lq = 128 * tiles - 60
+    edges = [Lq * i // groups + 17 * (0 < i < groups) for i in range(groups + 1)]
+    rects = [(a, b, 0, Lk * (i + 1) // groups) for i, (a, b) in enumerate(zip(edges, edges[1:]))]
+    rects += [(a, b, Lk - 40 * (i + 1), Lk - 5) for i, (a, b) in enumerate(zip(edges, edges[1:]))]
+    qr, kr = (torch.tensor([x[j:j + 2] for x in rects], dtype=torch.int32, device=gpu) for j in (0, 2))
+    mask = mm.prepare_magi_csr_and_tasks(qr, kr, Q_real=Lq, KV_real=Lk)
+    print(f"case split magi rounds B={B} H={H} D={D} kv={kv_tangents} {dtype}: {mask.T * B * H} tasks", flush=True)
+    code = nat.dtype_code(dtype)
+    assert mask.T * B * H > slots and nat.magi_split_bytes(code, mask.T, mask.key_tiles, B, H, D, D) > 0
+    q, k, v, tq, tk, tv = _draw(gpu, D, B, H, Lq, Lk, D, dtype)
+    tk, tv = (tk, tv) if kv_tangents else (None, None)
+    got, again = (jvp_attention_forward_magi(q, k, v, tq, tk, tv, D ** -0.5, mask) for _ in range(2))
+    whole = jvp_attention_forward_magi(q, k, v, tq, tk, tv, D ** -0.5, dataclasses.replace(mask, key_tiles=0))
+    torch.cuda.synchronize()
+    # every row against the launch that does not split (P~ rounded against another maximum: at most
+    # both errors, 2.4e-3 in bf16 and 3e-4 in fp16 each), and some rows of every group, in the first
+    # and the last head, against the oracle
+    rows = torch.cat([torch.arange(a, b, 61) for a, b in zip(edges, edges[1:])])
+    allow = torch.zeros(len(rows), Lk, dtype=torch.bool)
+    for a, b, s, e in rects:
+        allow[(rows >= a) & (rows < b), s:e] = True
+    zeros = torch.zeros_like(k)
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        xs = [(zeros if t is None else t)[b:b + 1, h:h + 1].cpu() for t in (q, k, v, tq, tk, tv)]
+        xs[0], xs[3] = xs[0][:, :, rows], xs[3][:, :, rows]
+        ref = om.masked_jvp(*xs, allow, D ** -0.5)
+        for name, a, w, r in zip(("o", "to", "lse", "mu"), got, whole, ref):
+            _no_worse(name, a[b:b + 1, h:h + 1, rows], w[b:b + 1, h:h + 1, rows], r)
+    for name, a, c, w in zip(("o", "to", "lse", "mu"), got, again, whole):
+        assert torch.equal(a, c), name
+        for b in range(B):
+            for h in range(H):
+                assert orc.rel_l2(a[b, h].cpu(), w[b, h].cpu()) <= (6e-3 if dtype == torch.bfloat16 else 1e-3), (name, b, h)
