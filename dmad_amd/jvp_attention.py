@@ -310,6 +310,9 @@ def _pair(x, tx):
 
 
 _PLAIN_TENSORS = {torch.Tensor, torch.nn.Parameter, type(None)}
+_dispatch_modes, _function_mode = torch._C._len_torch_dispatch_stack, torch._C._is_torch_function_mode_enabled
+_functorch_stack, _tracing_state = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+_profiling, _data_ptr, _is_neg = torch.autograd._profiler_enabled, torch.Tensor.data_ptr, torch.Tensor.is_neg
 
 
 def _eager_call(*ts) -> bool:
@@ -323,17 +326,18 @@ def _eager_call(*ts) -> bool:
     torch.autograd.grad(is_grads_batched=True) and vectorized jacobians, a torch.Tensor
     outside functorch's stack whose data_ptr() raises (the dispatcher calls the op per
     cotangent). The op costs about 7 us of host time per call beyond the call it wraps
-    (15 us), this check 3 us for the six operands of a JVP call."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
-            or torch._C._is_torch_function_mode_enabled() or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
-            or torch.autograd._profiler_enabled() or not _PLAIN_TENSORS.issuperset(map(type, ts))):
+    (15 us), this check 2 us for the six operands of a JVP call."""
+    if (torch.compiler.is_compiling() or _dispatch_modes() or _function_mode() or _functorch_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0 or _tracing_state() is not None
+            or _profiling() or not _PLAIN_TENSORS.issuperset(map(type, ts))):
         return False
-    ts = [t for t in ts if t is not None]
     try:
-        return all(map(torch.Tensor.data_ptr, ts)) and not any(map(torch.Tensor.is_neg, ts))
+        for t in ts:
+            if t is not None and (not _data_ptr(t) or _is_neg(t)):
+                return False
     except RuntimeError:
         return False
+    return True
 
 
 def _fwd_ws_bytes(dtype, mode, B, H, Lk, Dqk, Dv) -> int:
