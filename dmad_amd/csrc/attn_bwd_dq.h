@@ -565,7 +565,8 @@ struct DqTrCfg {
 // the third wave hides more of the 6 VALU instructions per MFMA (1% faster at
 // B=4, H=32, L=16384 than two waves at 172 VGPRs, with bitwise equal dQ).
 // SPLIT: the last work items run in pieces of the keys (split.h), each writing
-// its dQ accumulators as partials.
+// its dQ accumulators as partials. (At D = 64 one VGPR is spilled around the loop,
+// not in it.)
 template <typename T, int D, bool SPLIT = false>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 1) void attn_bwd_dq_tr_kernel(DqParams p) {
   using C = DqTrCfg<D>;

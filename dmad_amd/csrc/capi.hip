@@ -209,7 +209,8 @@ constexpr int64_t kX2MaxKeyTiles = 64;
 // train/wan/rcm/utils/flash_attention_jvp_triton.py:98-107). Its keys are the
 // dtype, the mode, the mask, Lq (query tiles per head), Lk (key tiles) and the
 // head dims; the entry points launch what it says, and dmad_attn_fwd_plan /
-// dmad_attn_bwd_plan report it. Inputs are validated by the callers.
+// dmad_attn_bwd_plan report it. Given scratch for partials the last tiles may run in
+// pieces instead (plan_fwd_split and the like below). Inputs are validated by the callers.
 enum class FwdFamily { kRows, kRowsX2, kGeneric, kF32 };
 struct FwdPlan {
   FwdFamily family;

@@ -9,8 +9,9 @@
 // into `n` pieces along its loop. A piece writes its fp32 accumulators to a
 // partial buffer, and a second, small kernel sums an item's pieces in a fixed
 // order (no atomics: repeated calls agree bit for bit) and writes the outputs.
-// What a launch does is decided once per shape on the host (plan_split) from the
-// items, the steps of an item's loop and the costs of the kernel that runs it.
+// What a launch does is decided on the host, on every call (plan_split, 0.1-0.7 us),
+// as a function of the items, the steps of an item's loop and the costs of the kernel
+// that runs it alone.
 #pragma once
 #include <type_traits>
 #include "common.h"
@@ -70,7 +71,10 @@ __device__ __forceinline__ f32x4_t split_get(const float* tile, int lane, int g)
 }
 
 // ---------------------------------------------------------------- host: the plan
-// Costs of one kernel of a split launch, in microseconds on an MI355X.
+// Costs of one kernel of a split launch, in microseconds on an MI355X whose clock the
+// power limit does not lower: those of launches of a few rounds. Long launches take
+// longer (the 64-wide query pass of 4 x 32 heads of 2048 tokens 201 us, 149 by its
+// costs), so that what a split of theirs saves is overrated by as much.
 struct SplitCost {
   int occ;          // workgroups that fit a CU
   float step;       // one step of the loop, one workgroup per CU
@@ -144,7 +148,8 @@ inline SplitPlan split_cut(int64_t items, int64_t rest, int n, int len, int64_t 
 
 // How to run `items` work items of `steps` steps: in full rounds, then the rest in
 // the pieces that finish soonest by the costs above (even_only: in pieces of one
-// length), where that saves at least a twentieth of the launch and 8 us: the second
+// length), where that saves at least a twentieth of the launch and 8 us (of a backward
+// in several launch pairs: of all pairs, of which only the last is cut): the second
 // kernel and its scratch cost the host 4-5 us, and calls that short wait for the
 // host (a training call of two 64-wide heads of 999 tokens: 45 us of kernels split,
 // 67 whole, in 200 us of host time, 12 of them for the three splits). The partials

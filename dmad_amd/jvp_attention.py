@@ -171,8 +171,9 @@ def _backward_workspace(code: int, ws_mode: int, B: int, H: int, Lq: int, Lk: in
 
 
 def _split_workspace(nbytes: int, device):
-    """(pointer, size, owner) of the partials of a split launch. The split only saves time:
-    without room for its partials (at most 128 MiB) every tile runs whole."""
+    """(pointer, size, owner) of the partials of a split launch (at most 128 MiB). Without room
+    for them every tile runs whole: slower, and sums are rounded in another order, so that such
+    a call's outputs differ in their last bits from those of one that had the room."""
     if nbytes == 0:
         return None, 0, None
     try:
@@ -206,7 +207,8 @@ def backward_plan(dtype: torch.dtype, B: int, H: int, Lq: int, Lk: int, D: int, 
                   tangent_grads: bool = False) -> dict:
     """The launch plan of the backward this op runs for these sizes under the current score
     budget (no GPU needed): kernels, grids, workspace and ``score_slices``; with score slices
-    the key and query passes run ``pairs`` times, one pair per group of slices."""
+    the key and query passes run ``pairs`` times, one pair per group of slices. Grids are those
+    of whole tiles: a pass whose last tiles run in pieces has more workgroups."""
     code = nat.dtype_code(dtype)
     mode = (2 if tangent_grads else 1) if full else 0
     ws = nat.bwd_workspace_bytes_of(code, mode, B, H, Lq, Lk, D) + _score_bytes(code, full, B, H, Lq, Lk, D)

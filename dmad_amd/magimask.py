@@ -262,7 +262,8 @@ class MagiMask:
     T: int
     BLOCK_M: int
     # most 32-key tiles a query group walks (0: not known): what the launch goes by when it
-    # decides whether to cut the last tasks; results do not depend on it
+    # decides whether to cut the last tasks, and into how many pieces (a cut task's outputs
+    # are the same but for their rounding)
     key_tiles: int = 0
 
 

@@ -5,8 +5,9 @@ teacher, the fake-score network and the critics call (through
 ``FlexOrSdpaLocalAttention`` in dense mode, blockmask.py:354-355, and
 wan2pt1.py:245, 281) and which picks FA3 / cuDNN / flash / efficient SDPA by
 GPU generation. Here it is one path: the plain forward kernel and the dO-only
-backward kernels, as the registered op ``dmad::flash_attn_fwd`` (so selective
-activation checkpointing keeps its output).
+backward kernels. Ordinary eager calls launch them directly; under anything
+that watches operators (selective activation checkpointing, which keeps their
+output, compilers, traces) they run as the registered op ``dmad::flash_attn_fwd``.
 """
 from __future__ import annotations
 

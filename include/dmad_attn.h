@@ -91,8 +91,9 @@ int dmad_attn_fwd_split_bytes(int dtype, int mode, int64_t B, int64_t H, int64_t
  * dmad_attn_jvp_fwd with a second scratch buffer (256-byte aligned). Query
  * tiles that do not fill a round over the chip are cut along their keys; the
  * pieces' fp32 results go to split_ws and are combined, in a fixed order, by
- * a second kernel. With split_ws null or smaller than
- * dmad_attn_fwd_split_bytes it is dmad_attn_jvp_fwd.
+ * a second kernel: O, Od, LSE and mu agree with dmad_attn_jvp_fwd's to
+ * rounding, and from call to call bit for bit. With split_ws null or smaller
+ * than dmad_attn_fwd_split_bytes it is dmad_attn_jvp_fwd.
  */
 int dmad_attn_jvp_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t Dqk, int64_t Dv,
                             const void* q, const void* k, const void* v, const void* tq, const void* tk,
@@ -133,8 +134,8 @@ int dmad_attn_jvp_fwd_magi(int dtype, int mode, int64_t B, int64_t H, int64_t Lq
  * dmad_attn_jvp_fwd_magi with scratch for partials, as dmad_attn_jvp_fwd_split:
  * the tasks that do not fill a round over the chip are cut into equal shares of
  * the key tiles each walks. key_tiles is the most 32-key tiles a task walks (it
- * decides whether and how far to cut, not what is computed; 0: not known, no
- * task is cut).
+ * decides whether to cut and into how many pieces, and so the rounding of the
+ * cut tasks' outputs, nothing else; 0: not known, no task is cut).
  */
 int dmad_attn_magi_split_bytes(int dtype, int64_t tasks, int64_t key_tiles, int64_t B, int64_t H, int64_t Dqk,
                                int64_t Dv, size_t* bytes);
@@ -270,7 +271,9 @@ int dmad_rmsnorm_rope_jvp(int dtype, int64_t rows, int64_t L, int64_t H, int64_t
  * Lk and the head dims -- where the reference autotunes its Triton forward
  * over 48 configs keyed on (SEQ_LEN_Q, SEQ_LEN_KV, HEAD_DIM_QK, HEAD_DIM_V)
  * (train/wan/rcm/utils/flash_attention_jvp_triton.py:98-107). The entry points
- * launch what the plan reports. Kernel names are static strings.
+ * launch what the plan reports, on whole tiles; the _split entry points, given
+ * their scratch, may run the last tiles in pieces (B and H then count, too),
+ * which the plan does not show. Kernel names are static strings.
  */
 typedef struct dmad_plan {
   const char* kernel;        /* forward kernel; backward: key-stationary pass (dK, dV) */
