@@ -168,14 +168,13 @@ __global__ __launch_bounds__(256, DH == 64 ? (MODE == kFwdPlain && !MAGI ? 4 : 2
   int skip = 0;               // MAGI, SPLIT: tiles of the task before this piece
   static_assert(!SPLIT || (C::CHUNKS == 1 && DVC == D), "split launches: all of V in one workgroup");
   if constexpr (SPLIT && MAGI) {
-    // Whole tasks: contiguous per XCD, or, where a head spans several XCDs (whose
-    // shares of a causal mask's growing tasks then differ widely), dealt over all of
-    // them from the last task down: two heads of a causal mask of 200 tasks 1.54 ->
-    // 1.18 ms, of teacher forcing 667 -> 607 us; five heads gained 5% and lost 5%.
-    const bool dealt = p.B * p.H <= 4;
-    SplitWork w = split_work(p.sp, !dealt, 0);
+    // Whole tasks (up to three heads, plan_magi_split) are dealt over all XCDs from
+    // the last one down: a head spans several XCDs, whose contiguous shares of a
+    // causal mask's growing tasks would differ widely (two heads of a causal mask of
+    // 200 tasks 1.54 -> 1.18 ms, of teacher forcing 667 -> 607 us).
+    SplitWork w = split_work(p.sp, 0, 0);
     if (w.item < 0) return;
-    if (dealt && w.piece < 0) w.item = p.sp.whole - 1 - w.item;
+    if (w.piece < 0) w.item = p.sp.whole - 1 - w.item;
     bh = w.item / p.T;
     const MagiTask t = magi_task(p, w.item - bh * p.T, C::BM);
     qt = t.row0 / C::BM;

@@ -313,12 +313,26 @@ dmad::SplitPlan plan_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_
 // see: `key_tiles`, the most 32-key tiles one of them walks, says what a split saves
 // (0: unknown, none). Each split task is cut in equal shares of its own tiles. As
 // the dense forward, both modes split alike.
+// Tasks that fit the chip at once all run in pieces (570 masks, one to forty heads:
+// 1.02-2.9 times as fast). Beyond that a plan in rounds misjudges tasks of unequal
+// lengths, and the whole ones keep their order, contiguous per XCD, which is the
+// better the more heads there are. Of 600 masks, block-causal and teacher-forcing
+// ones, a split was: one to three heads 1.04-1.74 times as fast (with the whole tasks
+// dealt, attn_fwd32_kernel; 0.86-0.99 where fewer than a 32nd of a round was left to
+// cut); four heads 0.81-1.46; five to seven 0.77-1.42; eight and more 0.81-1.31, the
+// middle below 1. So: up to three heads, and a 32nd of a round. Short walks stay whole,
+// too: a call that splits keeps the host busy for 25 us, as long as the kernel takes
+// without K, V tangents for 24 key tiles of 128-wide heads (24.6 us whole, 24.7-25.4
+// split; 26 tiles 26.5 and 24.8) and 36 of 64-wide ones (24.6 and 24.8; 41: 29.6 and 24.9).
 dmad::SplitPlan plan_magi_split(int dtype, int64_t tasks, int64_t key_tiles, int64_t B, int64_t H, int64_t Dqk,
                                 int64_t Dv) {
   dmad::SplitPlan none;
   none.whole = none.grid = tasks * B * H;
   if (dtype == DMAD_F32 || key_tiles <= 0 || !dmad::fwd32_supported((int)Dqk, (int)Dv)) return none;
-  return dmad::plan_split(tasks * B * H, key_tiles, fwd_split_cost(DMAD_FWD_JVP, Dqk), true);
+  if (key_tiles <= (Dqk == 128 ? 24 : 36)) return none;
+  const dmad::SplitCost cost = fwd_split_cost(DMAD_FWD_JVP, Dqk);
+  const dmad::SplitPlan pl = dmad::plan_split(tasks * B * H, key_tiles, cost, true);
+  return pl.whole > 0 && (B * H > 3 || pl.rest < dmad::kSplitCus * cost.occ / 32) ? none : pl;
 }
 
 dmad::FwdLaunchFn pick_fwd_magi_split(int dtype, int64_t d, int mode) {

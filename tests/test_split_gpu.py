@@ -283,12 +283,12 @@ def test_split_block_sparse_forward(gpu, hint, kv_tangents, D, dtype):
         assert torch.equal(a[:, :, 330:400], w[:, :, 330:400]), name  # no keys: zeros, LSE -inf
 
 
-@pytest.mark.parametrize("B,H,D,dtype", [(1, 2, 128, torch.bfloat16), (2, 2, 128, torch.float16), (1, 5, 128, torch.bfloat16),
-                                         (1, 4, 64, torch.bfloat16), (3, 2, 64, torch.float16)])
+@pytest.mark.parametrize("B,H,D,dtype", [(1, 2, 128, torch.bfloat16), (3, 1, 128, torch.float16), (1, 3, 64, torch.bfloat16),
+                                         (2, 1, 64, torch.float16)])
 @pytest.mark.parametrize("kv_tangents", [True, False])
 def test_split_block_sparse_forward_after_full_rounds(gpu, kv_tangents, B, H, D, dtype):
-    """Masks of more tasks than one round takes: whole tasks first (dealt over the chip from the last
-    one down up to four heads, contiguous per XCD beyond), then the rest in pieces."""
+    """Masks of more tasks than one round takes, up to three heads: whole tasks first, dealt over the
+    chip from the last one down, then the rest in pieces."""
     import dataclasses
 
     from dmad_amd import _native as nat
@@ -298,7 +298,7 @@ def test_split_block_sparse_forward_after_full_rounds(gpu, kv_tangents, B, H, D,
 
     slots = 256 if D == 128 else 512  # workgroups of a round
     groups, Lk = 8, 1700 if D == 128 else 3300
-    tiles = slots // (B * H) + 3  # query tiles of a head: a round and a few
+    tiles = (slots + slots // 16) // (B * H) + 1  # query tiles of a head: a round and a few
     Lq = 128 * tiles - 60
     edges = [Lq * i // groups + 17 * (0 < i < groups) for i in range(groups + 1)]
     rects = [(a, b, 0, Lk * (i + 1) // groups) for i, (a, b) in enumerate(zip(edges, edges[1:]))]

@@ -63,6 +63,22 @@ def test_pieces_fit_the_engines(L, pieces):
     assert nat.fwd_split_bytes(F32, JVP, 1, 12, L, L, 128, 128) == tiles * pieces * part
 
 
+@pytest.mark.parametrize("D,slots", [(64, 512), (128, 256)])
+def test_masks_split_where_their_tasks_fit_the_chip_or_belong_to_few_heads(D, slots):
+    """Tasks differ in length: with whole tasks in the launch a cut slows most masks of four and more
+    heads down, and those of fewer heads where hardly any task is left to cut; walks of 24 tiles are
+    over before the host has issued two launches."""
+    for BH in (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16, 20, 24, 40):
+        for tasks in range(1, 4 * slots // BH + 2):
+            items, rest = tasks * BH, tasks * BH % slots
+            for kt in (24, 60, 200, 500):
+                if kt == 24 or (items > slots and (BH > 3 or rest < slots // 32)):
+                    assert nat.magi_split_bytes(BF16, tasks, kt, 1, BH, D, D) == 0, (BH, tasks, kt)
+    assert nat.magi_split_bytes(BF16, slots // 4, 200, 1, 1, D, D) > 0
+    assert nat.magi_split_bytes(BF16, slots // 128, 200, 2, 12, D, D) > 0
+    assert nat.magi_split_bytes(BF16, slots // 3 + 7, 200, 3, 1, D, D) > 0
+
+
 def test_argument_checks():
     with pytest.raises(ValueError):
         nat.fwd_split_bytes(BF16, JVP, 1, 2, 64, 64, 96, 96)
