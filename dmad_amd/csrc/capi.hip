@@ -319,8 +319,8 @@ dmad::SplitPlan plan_fwd_split(int dtype, int mode, int64_t B, int64_t H, int64_
 // better the more heads there are. Of 600 masks, block-causal and teacher-forcing
 // ones, a split was: one to three heads 1.04-1.74 times as fast (with the whole tasks
 // dealt, attn_fwd32_kernel; 0.86-0.99 where fewer than a 32nd of a round was left to
-// cut); four heads 0.81-1.46; five to seven 0.77-1.42; eight and more 0.81-1.31, the
-// middle below 1. So: up to three heads, and a 32nd of a round. Short walks stay whole,
+// cut); four heads 0.81-1.46; five to seven 0.77-1.42; eight and more 0.81-1.31, mostly
+// below 1. So: up to three heads, and a 32nd of a round. Short walks stay whole,
 // too: a call that splits keeps the host busy for 25 us, as long as the kernel takes
 // without K, V tangents for 24 key tiles of 128-wide heads (24.6 us whole, 24.7-25.4
 // split; 26 tiles 26.5 and 24.8) and 36 of 64-wide ones (24.6 and 24.8; 41: 29.6 and 24.9).
