@@ -182,6 +182,20 @@ def _split_workspace(nbytes: int, device):
         return None, 0, None
 
 
+def _backward_scratch(code: int, ws_mode: int, B: int, H: int, Lq: int, Lk: int, D: int, device):
+    """The partials and the workspace of a backward, (pointer, size, owner) each. The partials
+    first: without room for them every gradient's last bits change, without room for the
+    stored scores none do. Where the minimum workspace then does not fit, the partials go."""
+    split = _split_workspace(nat.bwd_split_bytes(code, ws_mode > 0, ws_mode == 2, B, H, Lq, Lk, D), device)
+    try:
+        return split, _backward_workspace(code, ws_mode, B, H, Lq, Lk, D, device)
+    except torch.cuda.OutOfMemoryError:
+        if split[2] is None:
+            raise
+    split = None, 0, None
+    return split, _backward_workspace(code, ws_mode, B, H, Lq, Lk, D, device)
+
+
 def _score_slices(bh: int, n_max: int, Lq: int, Lk: int) -> int:
     """(b, h) slices per launch pair, at most n_max: the count whose pairs fill the 256 CUs
     best. A pair of n slices runs n * key tiles key-pass workgroups and n * query-block
@@ -505,10 +519,7 @@ def jvp_attention_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dout, dto, sm_sc
     dtv = torch.empty_like(dv) if tgrads else None
     lib = nat.lib()
     ws_mode = (2 if tgrads else 1) if full else 0
-    # the partials first: without room for them every gradient's last bits change, without
-    # room for the stored scores none do
-    sp_ptr, sp_size, sp = _split_workspace(nat.bwd_split_bytes(code, full, tgrads, B, H, Lq, Lk, D), q.device)
-    ws_ptr, ws_size, ws = _backward_workspace(code, ws_mode, B, H, Lq, Lk, D, q.device)
+    (sp_ptr, sp_size, sp), (ws_ptr, ws_size, ws) = _backward_scratch(code, ws_mode, B, H, Lq, Lk, D, q.device)
     nat.check(
         lib.dmad_attn_jvp_bwd_split(
             code, B, H, Lq, Lk, D,

@@ -315,3 +315,40 @@ def test_backward_workspace_falls_back_to_the_minimum(monkeypatch):
     monkeypatch.setattr(ja.nat, "workspace", lambda n, d: fake_workspace(n, d, limit=0))
     with pytest.raises(torch.cuda.OutOfMemoryError):
         ja._backward_workspace(BF16, 0, 1, 40, 32760, 32760, 128, "cpu")
+
+
+def test_backward_scratch_gives_up_what_it_can_do_without(monkeypatch):
+    """With less and less memory: the stored scores go first, then the partials of a split launch,
+    and only a minimum workspace that does not fit by itself fails."""
+    import weakref
+
+    from dmad_amd import jvp_attention as ja
+
+    shape = (1, 12, 6240, 6240, 128)
+    part = ja.nat.bwd_split_bytes(BF16, False, False, *shape)
+    base, extra = ja.nat.bwd_workspace_bytes_of(BF16, 0, *shape), ja._score_bytes(BF16, False, *shape)
+    assert part > 0 and extra > 0
+
+    class Block:
+        pass
+
+    live = weakref.WeakKeyDictionary()
+
+    def pool(capacity):
+        def workspace(nbytes, device):
+            if sum(live.values()) + nbytes > capacity:
+                raise torch.cuda.OutOfMemoryError("no room")
+            block = Block()
+            live[block] = nbytes
+            return 1 << 20, nbytes, block
+        return workspace
+
+    for capacity, want in ((part + base + extra, (part, base + extra)), (part + base + extra - 1, (part, base)),
+                           (part + base, (part, base)), (part + base - 1, (0, base)), (base, (0, base))):
+        monkeypatch.setattr(ja.nat, "workspace", pool(capacity))
+        split, ws = ja._backward_scratch(BF16, 0, *shape, "cpu")
+        assert (split[1], ws[1]) == want, capacity
+        del split, ws
+    monkeypatch.setattr(ja.nat, "workspace", pool(base - 1))
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        ja._backward_scratch(BF16, 0, *shape, "cpu")
